@@ -12,12 +12,14 @@
 //  * gemm_skinny — N <= 64 tokens (the 48-token action expert): HBM-bound
 //                  weight streaming with MFMA 16x16x32, K split across the
 //                  waves of a workgroup and reduced in LDS.
-//  * gemm_simt   — f32 weights (generic MUL_MAT only), plain FMA.
+//  * gemm_f32    — f32 weights (the f32 reference profile, generic MUL_MAT),
+//                  f32 MFMA 16x16x4.
 #include "../internal.h"
 #include "device.h"
 #include "rowops.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace wamx {
@@ -1732,6 +1734,16 @@ static void launch_skinny_wk(const GemmParams & p, hipStream_t s) {
     }
 }
 
+static void launch_reduce(const GemmParams & p, const float * part, int splits, hipStream_t s) {
+    const int64_t total = p.N * p.M;
+    if (p.M % 4 == 0)
+        hipLaunchKernelGGL(gemm_skinny_reduce<4>, dim3((unsigned) ((total / 4 + 255) / 256)), dim3(256), 0, s, p, part,
+                           splits);
+    else
+        hipLaunchKernelGGL(gemm_skinny_reduce<1>, dim3((unsigned) ((total + 255) / 256)), dim3(256), 0, s, p, part,
+                           splits);
+}
+
 static hipError_t run_skinny(const GemmParams & p, bool xf32, bool tiled, void * ws, size_t ws_bytes, hipStream_t s) {
     if (skinny_wk_ok(p, xf32, tiled) && skinny_wk_enabled()) {
         switch ((p.N + 15) / 16) {
@@ -1748,33 +1760,159 @@ static hipError_t run_skinny(const GemmParams & p, bool xf32, bool tiled, void *
         return hipErrorInvalidValue;
     float * part = splits > 1 ? (float *) ws : nullptr;
     launch_skinny_part(p, xf32, tiled, part, splits, ks, waves, s);
-    if (splits > 1) {
-        const int64_t total = p.N * p.M;
-        if (p.M % 4 == 0)
-            hipLaunchKernelGGL(gemm_skinny_reduce<4>, dim3((unsigned) ((total / 4 + 255) / 256)), dim3(256), 0, s, p,
-                               (const float *) part, splits);
-        else
-            hipLaunchKernelGGL(gemm_skinny_reduce<1>, dim3((unsigned) ((total + 255) / 256)), dim3(256), 0, s, p,
-                               (const float *) part, splits);
-    }
+    if (splits > 1) launch_reduce(p, part, splits, s);
     return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
-// gemm_simt: f32 weights (generic MUL_MAT of two f32 tensors, not on the
-// native bf16 path).  One thread per output, fp32 FMA over K.
+// gemm_f32: f32 weights (the f32 reference profile, MUL_MAT of two f32
+// tensors, f32 convolutions), products and sums in f32 on MFMA 16x16x4.
+//
+// The f32 matrix rate is 1/16 of bf16's (154 TFLOP/s measured on a large
+// product), so the tile needs little LDS bandwidth and the work is bound by
+// the MFMAs at 48 or more tokens and by the weight stream below that.  A
+// workgroup of 4 waves multiplies 16 NT tokens by 64 RG features; K steps of
+// 32 go through two LDS stages with the next step's loads held in registers
+// meanwhile.  In a step, lane group g's 16-byte fragment covers columns 16 q +
+// 4 g .. + 4 of both operands and feeds 4 MFMAs, one column of each group per
+// MFMA (both operands take the same K order, so any order is a valid one).
+// Rows are padded by 4 floats: 16 rows' 16-byte reads cover all 64 banks.
+// K slices (blockIdx.y) write f32 partials that gemm_skinny_reduce sums in
+// slice order.
+// One thread per output with a serial K loop, which this replaced, took
+// 1998 us for 3072 x 48 x 3072 and 9287 us for 14336 x 48 x 3072; now 27 and
+// 67 us (1.4 and 2.6 TB/s of weights), and its error against 64-bit sums over
+// an action layer is a third of the serial sum's.
+// VEC: rows start at 16-byte multiples and K % 4 == 0; else scalar loads of
+// 32 consecutive columns per half wave.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void gemm_simt(GemmParams p, int32_t x_type) {
-    const int64_t m = (int64_t) blockIdx.x * 256 + threadIdx.x;
-    const int64_t n = blockIdx.y;
-    const int64_t bz = blockIdx.z, b2 = bz % p.B2, b3 = bz / p.B2;
-    if (m >= p.M) return;
-    const float * w = (const float *) p.w + (b2 / p.r2) * p.w_bs2 + (b3 / p.r3) * p.w_bs3 + m * p.ldw;
-    const int64_t xo = b2 * p.x_bs2 + b3 * p.x_bs3 + n * p.ldx;
-    float acc = 0.0f;
-    for (int64_t k = 0; k < p.K; ++k) acc = fmaf(w[k], load_as_f32(p.x, x_type, xo + k), acc);
+constexpr int kF32BK = 32, kF32Pitch = kF32BK + 4, kF32Threads = 256;
+
+template <int NT, int RG, bool VEC, bool XBF>
+__global__ __launch_bounds__(kF32Threads) void gemm_f32(GemmParams p, float * part, int nt_m, int nt_n, int ks) {
+    constexpr int BM = 16 * NT, BN = 64 * RG, ROWS = BM + BN;
+    constexpr int PER = ROWS * kF32BK / 4 / kF32Threads;  // 16-byte chunks per thread per step
+    constexpr int RPC = kF32Threads / 8;                  // rows per chunk instruction
+    constexpr int LEFT = ROWS - PER * RPC;                // rows of a last part-full instruction
+    constexpr int NL = PER + (LEFT > 0);
+    static_assert(!(VEC && XBF), "bf16 activations take the scalar loads");
+    __shared__ __align__(16) float st[2][ROWS * kF32Pitch];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int g = lane >> 4, r16 = lane & 15;
+    const int64_t b2 = blockIdx.z % p.B2, b3 = blockIdx.z / p.B2;
+    const float * w = (const float *) p.w + (b2 / p.r2) * p.w_bs2 + (b3 / p.r3) * p.w_bs3;
+    const char * x = (const char *) p.x + (b2 * p.x_bs2 + b3 * p.x_bs3) * (XBF ? 2 : 4);
+    int tm, tn;
+    tile_coords((int) blockIdx.x, nt_m, nt_n, tm, tn);
+    const int64_t n0 = (int64_t) tn * BM, m0 = (int64_t) tm * BN;
+    const int64_t kb = (int64_t) blockIdx.y * ks;
+    const int klen = (int) min(p.K - kb, (int64_t) ks);
+    const int nsteps = (klen + kF32BK - 1) / kF32BK;
+
+    // A load instruction takes 32 rows (VEC: 8 threads of 4 columns a row) or 8
+    // (32 threads of one column a row).
+    float4 rv[VEC ? NL : 1];
+    float rs[VEC ? 1 : 4 * NL];
+    // Sources are byte offsets from the tile's first token and weight row,
+    // so a step adds one offset to each.
+    const char * xt = x + (n0 * p.ldx + kb) * (XBF ? 2 : 4);
+    const char * wt = (const char *) (w + m0 * p.ldw + kb);
+    constexpr int RPI = VEC ? RPC : RPC / 4, NI = VEC ? NL : 4 * NL;
+    const int64_t ldx = p.ldx, ldw = p.ldw;
+    const int nlast = (int) min(p.N - n0, (int64_t) BM) - 1, mlast = (int) min(p.M - m0, (int64_t) BN) - 1;
+    const char * src[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int r = min(i * RPI + tid / (VEC ? 8 : 32), ROWS - 1);
+        const char * xr = xt + (int64_t) min(r, nlast) * ldx * (XBF ? 2 : 4);
+        const char * wr = wt + (int64_t) min(max(r - BM, 0), mlast) * ldw * 4;
+        src[i] = r < BM ? xr : wr;
+    }
+    auto load = [&](int step) {
+        if constexpr (VEC) {
+            const int k = step * kF32BK + 4 * (tid & 7), kc = min(k, klen - 4);
+#pragma unroll
+            for (int i = 0; i < NL; ++i) {
+                rv[i] = *(const float4 *) (src[i] + (int64_t) kc * 4);
+            }
+        } else {
+            const int k = step * kF32BK + (tid & 31), kc = min(k, klen - 1);
+#pragma unroll
+            for (int i = 0; i < 4 * NL; ++i) {
+                // BM is a multiple of the rows of an instruction: all of them tokens, or all weights.
+                if (XBF && i * RPI < BM) rs[i] = bf16_to_f32(*(const uint16_t *) (src[i] + (int64_t) kc * 2));
+                else rs[i] = *(const float *) (src[i] + (int64_t) kc * 4);
+            }
+        }
+    };
+    // The K tail is zeroed here and not at the load: a use of a loaded register
+    // right after its load would make the wave wait for it before the MFMAs.
+    auto store = [&](int step, float * s) {
+        if constexpr (VEC) {
+            const bool ok = step * kF32BK + 4 * (tid & 7) < klen;
+#pragma unroll
+            for (int i = 0; i < NL; ++i) {
+                const int r = i * RPC + (tid >> 3);
+                if (i < PER || r < ROWS)
+                    *(float4 *) (s + r * kF32Pitch + 4 * (tid & 7)) = ok ? rv[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+        } else {
+            const bool ok = step * kF32BK + (tid & 31) < klen;
+#pragma unroll
+            for (int i = 0; i < 4 * NL; ++i) {
+                const int r = i * (RPC / 4) + (tid >> 5);
+                if (i < 4 * PER || r < ROWS) s[r * kF32Pitch + (tid & 31)] = ok ? rs[i] : 0.0f;
+            }
+        }
+    };
+
+    f32x4_t acc[RG][NT];
+#pragma unroll
+    for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[rg][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    load(0);
+    store(0, st[0]);
+    __syncthreads();
+    for (int step = 0; step < nsteps; ++step) {
+        if (step + 1 < nsteps) load(step + 1);
+        const float * cur = st[step & 1];
+#pragma unroll
+        for (int q = 0; q < kF32BK / 16; ++q) {
+            f32x4_t wa[RG], xa[NT];
+#pragma unroll
+            for (int rg = 0; rg < RG; ++rg)
+                wa[rg] = *(const f32x4_t *) (cur + (BM + 16 * (RG * wave + rg) + r16) * kF32Pitch + 16 * q + 4 * g);
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                xa[t] = *(const f32x4_t *) (cur + (16 * t + r16) * kF32Pitch + 16 * q + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+                        acc[rg][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[t][e], wa[rg][e], acc[rg][t], 0, 0, 0);
+        }
+        if (step + 1 < nsteps) store(step + 1, st[(step + 1) & 1]);
+        __syncthreads();
+    }
     char * y = (char *) p.y + (b2 * p.y_bs2 + b3 * p.y_bs3) * (p.y_type == WAMX_TYPE_F32 ? 4 : 2);
-    store_out(p, y, p.res, n, m, acc);
+    float * pp = part ? part + (int64_t) blockIdx.y * p.N * p.M : nullptr;
+#pragma unroll
+    for (int rg = 0; rg < RG; ++rg) {
+        const int64_t m = m0 + 16 * (RG * wave + rg) + r16;
+        if (m >= p.M) continue;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t n = n0 + 16 * t + 4 * g + r;
+                if (n >= p.N) continue;
+                if (pp) pp[n * p.M + m] = acc[rg][t][r];
+                else store_out(p, y, p.res, n, m, acc[rg][t][r]);
+            }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1894,13 +2032,7 @@ static void launch_dma_splitk_parts(const GemmParams & p, int splits, void * ws,
 }
 static hipError_t run_dma_splitk(const GemmParams & p, int splits, void * ws, hipStream_t s) {
     launch_dma_splitk_parts(p, splits, ws, s);
-    const int64_t total = p.N * p.M;
-    if (p.M % 4 == 0)
-        hipLaunchKernelGGL(gemm_skinny_reduce<4>, dim3((unsigned) ((total / 4 + 255) / 256)), dim3(256), 0, s, p,
-                           (const float *) ws, splits);
-    else
-        hipLaunchKernelGGL(gemm_skinny_reduce<1>, dim3((unsigned) ((total + 255) / 256)), dim3(256), 0, s, p,
-                           (const float *) ws, splits);
+    launch_reduce(p, (const float *) ws, splits, s);
     return hipGetLastError();
 }
 
@@ -2148,17 +2280,82 @@ __global__ void round_rows_bf16_kernel(const float * __restrict__ x, int64_t ldx
     *(uint4 *) (y + r * K + 8 * c) = pack8(v);
 }
 
+// Tile and K split of an f32 product: the tokens in blocks of 16 NT with the
+// least padding, then the feature block (64 or 128) and the slice count with
+// the least modelled time, in us.  A workgroup's K step costs its MFMAs (32
+// cycles each on its SIMD) or its share of the weight stream, and 0.6 of load
+// latency that only a second workgroup of the CU hides; a split adds the
+// partials' traffic and the reduce.  Weights from HBM, sweep of both
+// parameters: 3072 x 48 x 3072 26.8 us in 16 slices of 64 features against
+// 32.6 in 5, 14336 x 48 x 3072 67 in 3 or 4 slices against 92 unsplit, 3072 x
+// 121 x 3072 45 in 10 slices against 55 in 20; the model's choice is within a
+// tenth of each shape's best (times with a graph launch of one node).
+static void f32_plan(const GemmParams & p, bool may_split, size_t ws_bytes, int & nt, int & rg, int & splits, int & ks) {
+    if (p.N <= 64) nt = (int) ((p.N + 15) / 16);
+    else nt = (p.N + 127) / 128 * 128 > (p.N + 63) / 64 * 64 ? 4 : 8;
+    const int64_t steps = (p.K + kF32BK - 1) / kF32BK;
+    const int64_t nb = (p.N + 16 * nt - 1) / (16 * nt);
+    double best = 1e30;
+    rg = nt == 8 ? 2 : 1;
+    splits = 1;
+    ks = (int) steps * kF32BK;
+    for (int r = nt == 8 ? 2 : 1; r <= 2; ++r)
+        for (int64_t sp = 1; sp <= (may_split ? 32 : 1); ++sp) {
+            const int64_t per = (steps + sp - 1) / sp, s = (steps + per - 1) / per;
+            if (s != sp || (sp > 1 && (per < 4 || (size_t) sp * p.N * p.M * sizeof(float) > ws_bytes))) continue;
+            const double wgs = (double) nb * (double) ((p.M + 64 * r - 1) / (64 * r)) * (double) sp;
+            const double step = std::max(0.12 * nt, 0.36) * r;
+            double t = (double) per * std::max(std::ceil(wgs / 256) * step, step + 0.6);
+            if (sp > 1) t += (double) sp * (double) p.N * (double) p.M * 8 / 4e6 + 3.0;
+            if (t < best) {
+                best = t;
+                rg = r;
+                splits = (int) sp;
+                ks = (int) per * kF32BK;
+            }
+        }
+}
+
+static hipError_t run_f32(const GemmArgs & a, const GemmParams & p, hipStream_t s) {
+    const bool xbf = a.x_type == WAMX_TYPE_BF16;
+    if (!xbf && a.x_type != WAMX_TYPE_F32) return hipErrorInvalidValue;
+    const bool vec = !xbf && a.K % 4 == 0 && a.ldw % 4 == 0 && a.ldx % 4 == 0 && aligned16(a.w) && aligned16(a.x) &&
+                     a.w_bs2 % 4 == 0 && a.w_bs3 % 4 == 0 && a.x_bs2 % 4 == 0 && a.x_bs3 % 4 == 0;
+    const int64_t batches = a.B2 * a.B3;
+    int nt, rg, splits, ks;
+    f32_plan(p, batches == 1 && a.ws && aligned16(a.ws), a.ws_bytes, nt, rg, splits, ks);
+    const int nt_m = (int) ((p.M + 64 * rg - 1) / (64 * rg)), nt_n = (int) ((p.N + 16 * nt - 1) / (16 * nt));
+    const dim3 grid((unsigned) (nt_m * nt_n), (unsigned) splits, (unsigned) batches);
+    float * part = splits > 1 ? (float *) a.ws : nullptr;
+#define WAMX_F32(NT, RG)                                                                                               \
+    do {                                                                                                               \
+        if (vec) hipLaunchKernelGGL((gemm_f32<NT, RG, true, false>), grid, dim3(kF32Threads), 0, s, p, part, nt_m, nt_n, ks); \
+        else if (xbf) hipLaunchKernelGGL((gemm_f32<NT, RG, false, true>), grid, dim3(kF32Threads), 0, s, p, part, nt_m, nt_n, ks); \
+        else hipLaunchKernelGGL((gemm_f32<NT, RG, false, false>), grid, dim3(kF32Threads), 0, s, p, part, nt_m, nt_n, ks); \
+    } while (0)
+    switch (nt * 2 + rg - 1) {
+        case 2: WAMX_F32(1, 1); break;
+        case 3: WAMX_F32(1, 2); break;
+        case 4: WAMX_F32(2, 1); break;
+        case 5: WAMX_F32(2, 2); break;
+        case 6: WAMX_F32(3, 1); break;
+        case 7: WAMX_F32(3, 2); break;
+        case 8: WAMX_F32(4, 1); break;
+        case 9: WAMX_F32(4, 2); break;
+        default: WAMX_F32(8, 2); break;
+    }
+#undef WAMX_F32
+    if (splits > 1) launch_reduce(p, part, splits, s);
+    return hipGetLastError();
+}
+
 hipError_t launch_gemm(const GemmArgs & a, hipStream_t s) {
     const GemmParams p = make_params(a);
     const int64_t batches = a.B2 * a.B3;
     if (a.M <= 0 || a.N <= 0 || batches <= 0) return hipSuccess;
     if (a.K <= 0) return hipErrorInvalidValue;
 
-    if (a.w_type == WAMX_TYPE_F32) {
-        dim3 grid((unsigned) ((a.M + 255) / 256), (unsigned) a.N, (unsigned) batches);
-        hipLaunchKernelGGL(gemm_simt, grid, dim3(256), 0, s, p, a.x_type);
-        return hipGetLastError();
-    }
+    if (a.w_type == WAMX_TYPE_F32) return run_f32(a, p, s);
     if (a.w_type != WAMX_TYPE_BF16 || (a.x_type != WAMX_TYPE_BF16 && a.x_type != WAMX_TYPE_F32))
         return hipErrorInvalidValue;
     const bool xf32 = a.x_type == WAMX_TYPE_F32;
