@@ -124,3 +124,30 @@ def test_f32_conv_batched_strided_dilated(wx, be, orc):
     got = r.fetch(y, np.float32, (2, 24, y.ne[1], y.ne[0]))
     ref = orc.conv_2d(k, x, 2, 2, 2, 2, 2, 2)
     assert np.allclose(got, ref, rtol=1e-4, atol=1e-4)
+
+
+# Edges of the implicit GEMM: channels below, at and past a 32-channel chunk
+# (and one channel); output channels of each tile width (160, 128, 64, 32)
+# with remainders; pixels below and past a 128-pixel tile; 1 x 1, strided,
+# dilated and unevenly padded windows; K slices (few pixels, many channels)
+# and none; several images; an image packed in several bands of rows.
+@pytest.mark.parametrize("IC,OC,KW,KH,s,p,d,IW,IH,B", [
+    (1, 1, 3, 3, (1, 1), (1, 1), (1, 1), 5, 4, 1), (3, 30, 3, 3, (1, 1), (1, 1), (1, 1), 65, 33, 2),
+    (33, 160, 3, 3, (2, 2), (0, 0), (1, 1), 41, 37, 1), (64, 130, 1, 1, (1, 1), (0, 0), (1, 1), 63, 9, 3),
+    (100, 200, 3, 2, (1, 2), (2, 1), (2, 1), 30, 29, 1), (640, 640, 3, 3, (1, 1), (1, 1), (1, 1), 15, 12, 1),
+    (160, 16, 5, 3, (3, 1), (4, 0), (1, 2), 70, 20, 2), (256, 32, 3, 3, (1, 1), (1, 1), (1, 1), 340, 280, 1)])
+def test_bf16_conv_integers_exact(wx, be, orc, IC, OC, KW, KH, s, p, d, IW, IH, B):
+    """Integer images and kernels: the f32 sum is exact, so the result is its
+    bf16 rounding whatever the order of summation."""
+    print(f"conv KAT {IC}->{OC} {KW}x{KH} s{s} p{p} d{d} at {IW}x{IH} x{B}", flush=True)
+    rng = np.random.default_rng(IC * OC + IW)
+    k = rng.integers(-4, 5, (OC, IC, KH, KW)).astype(np.float32)
+    x = rng.integers(-4, 5, (B, IC, IH, IW)).astype(np.float32)
+    r = Runner(wx, be, 1 << 28)
+    tk = r.leaf("bf16", (KW, KH, IC, OC), _bf(wx, k), "weight")
+    tx = r.leaf("bf16", (IW, IH, IC, B), _bf(wx, x), "input")
+    y = gm.conv_2d_direct(tk, tx, s[0], s[1], p[0], p[1], d[0], d[1])
+    r.run([y])
+    ref = orc.conv_2d(k, x, s[0], s[1], p[0], p[1], d[0], d[1])
+    assert ref.shape == (B, OC, y.ne[1], y.ne[0])
+    assert np.array_equal(r.fetch(y, np.uint16, ref.shape), _bf(wx, ref))

@@ -66,6 +66,10 @@ constexpr size_t kBackendWorkspaceBytes = 64ull << 20;
 // tokens, given ws_bytes of workspace; 0 when the product takes no K split.
 size_t linear_split_bytes(int64_t M, int64_t N, int64_t K, int32_t x_type, size_t ws_bytes);
 
+// y[n][m] (row stride ldy) = sum over splits of part[split][n][m], in split order.
+hipError_t launch_partial_sum(const float * part, int splits, int64_t N, int64_t M, void * y, int32_t y_type,
+                              int64_t ldy, hipStream_t s);
+
 // Row ops that consume a skinny GEMM's output, applied by its split-K reduce
 // in the same launch (one workgroup per token row).  The GEMM output itself
 // is still written.
@@ -164,8 +168,10 @@ hipError_t launch_rope_f32(const TensorRef & x, const int32_t * pos, const Tenso
 hipError_t launch_im2col(const TensorRef & src, const TensorRef & dst, int KW, int KH, int s0, int s1, int p0, int p1,
                          int d0, int d1, hipStream_t s);
 // ggml_conv_2d_direct (kernel [KW,KH,IC,OC], input [IW,IH,IC,N], dst
-// [OW,OH,OC,N]; pp = {s0, s1, p0, p1, d0, d1}): im2col row chunks in the
-// upper half of ws, the GEMM's partials in the lower half.
+// [OW,OH,OC,N]; pp = {s0, s1, p0, p1, d0, d1}).  bf16: implicit GEMM over the
+// image and kernel packed channels-last at the end of ws, f32 partials before
+// them.  f32: im2col row chunks in the upper half of ws, the GEMM's partials
+// in the lower half.
 hipError_t launch_conv2d(const TensorRef & kernel, const TensorRef & input, const TensorRef & dst, const int32_t * pp,
                          void * ws, size_t ws_bytes, hipStream_t s);
 hipError_t launch_modulation(const void * mod, int32_t mod_type, const void * tables, int32_t tab_type, float * out,

@@ -2349,6 +2349,18 @@ static hipError_t run_f32(const GemmArgs & a, const GemmParams & p, hipStream_t 
     return hipGetLastError();
 }
 
+hipError_t launch_partial_sum(const float * part, int splits, int64_t N, int64_t M, void * y, int32_t y_type,
+                              int64_t ldy, hipStream_t s) {
+    GemmParams p{};
+    p.y = y;
+    p.y_type = y_type;
+    p.ldy = ldy;
+    p.M = M;
+    p.N = N;
+    launch_reduce(p, part, splits, s);
+    return hipGetLastError();
+}
+
 hipError_t launch_gemm(const GemmArgs & a, hipStream_t s) {
     const GemmParams p = make_params(a);
     const int64_t batches = a.B2 * a.B3;
