@@ -3,9 +3,11 @@
 // GELU/GELU_ERF/SILU, CONCAT, GET_ROWS, SOFT_MAX, ROPE), the per-layer adaLN
 // modulation sum, and the seeded synthetic-weight generator.
 //
-// Tensors are 4-D strided views (ne[], byte strides nb[]); one thread per
-// destination element, index decomposed in ne[0]-fastest order so consecutive
-// threads touch consecutive destination elements.
+// Tensors are 4-D strided views (ne[], byte strides nb[]), walked in
+// ne[0]-fastest order so consecutive threads touch consecutive destination
+// elements.  The map kernel takes the usual forms (broadcast by whole dims, at
+// most 2^31 chunks) in 8, 4 or 1 elements per thread; the one-element kernels
+// with 64-bit index arithmetic take the rest.
 #include "../internal.h"
 #include "device.h"
 
@@ -70,6 +72,261 @@ __global__ void copy_kernel(Ref4 src, Ref4 dst, int64_t n) {
     } else {
         st(dst, pd, ld(src, ps));
     }
+}
+
+// ---------------------------------------------------------------------------
+// Strided map: copies and casts, ADD / MUL / REPEAT, unary ops and CONCAT over
+// dims merged where every operand allows it, V consecutive elements of dim 0
+// per thread.  The one-element kernels spend their time on three 64-bit
+// divisions per operand and element and on 2- or 4-byte accesses; here the
+// index takes at most three multiplications for 8 elements.  Measured: ADD of
+// a [192, 160, 160] bf16 image and a per-channel bias 31 -> 7.6 us, concatenation
+// of 9.6 M bf16 along dim 1 42 -> 9.5 us, along dim 0 at odd offsets (one
+// element per thread) 42 -> 26 us.
+// ---------------------------------------------------------------------------
+// n / d for n < 2^31 by a multiplication (Granlund and Montgomery, "Division by
+// Invariant Integers using Multiplication", 1994, figure 4.1: m' = floor(2^32
+// (2^l - d) / d) + 1 with l = ceil(log2 d), quotient (mulhi(m', n) + n) >> l;
+// the sum stays below 2^32 for such n).
+struct FastDiv {
+    uint32_t d, mul, shift;
+};
+static FastDiv fast_div(uint32_t d) {
+    uint32_t l = 0;
+    while ((1ull << l) < d) ++l;
+    return FastDiv{d, (uint32_t) ((((1ull << l) - d) << 32) / d + 1), l};
+}
+__device__ __forceinline__ uint32_t div(uint32_t n, const FastDiv & f) { return (__umulhi(f.mul, n) + n) >> f.shift; }
+
+struct MapOperand {
+    char * p;
+    int64_t s0, s1, s2, s3;  // byte strides; 0: broadcast
+    int32_t type;
+};
+struct MapArgs {
+    MapOperand a, b, d;
+    FastDiv n0, n1, n2;      // chunks of dim 0, elements of dims 1 and 2
+    uint32_t total;          // chunks
+    float scale, bias;
+    int32_t uop, dim;        // unary op; concatenated dim
+    uint32_t split;          // chunks (dim 0) or elements of it that come from a
+};
+enum { kMapCopy = 0, kMapAdd, kMapMul, kMapUnary, kMapConcat };
+
+template <int V>
+__device__ __forceinline__ void map_load(int32_t type, const char * p, int64_t s0, float (&o)[V]) {
+    if (V == 1 || s0 == 0) {
+        float v;
+        switch (type) {
+            case WAMX_TYPE_F32: v = *(const float *) p; break;
+            case WAMX_TYPE_BF16: v = bf16_to_f32(*(const uint16_t *) p); break;
+            case WAMX_TYPE_I32: v = (float) *(const int32_t *) p; break;
+            default: v = (float) *(const _Float16 *) p; break;
+        }
+#pragma unroll
+        for (int i = 0; i < V; ++i) o[i] = v;
+        return;
+    }
+    if constexpr (V > 1) {
+        uint32_t u[V];
+        if (type == WAMX_TYPE_F32 || type == WAMX_TYPE_I32) {
+#pragma unroll
+            for (int i = 0; i < V / 4; ++i) *(uint4 *) &u[4 * i] = ((const uint4 *) p)[i];
+#pragma unroll
+            for (int i = 0; i < V; ++i) o[i] = type == WAMX_TYPE_F32 ? __uint_as_float(u[i]) : (float) (int32_t) u[i];
+        } else {
+            if constexpr (V == 8) *(uint4 *) u = *(const uint4 *) p;
+            else *(uint2 *) u = *(const uint2 *) p;
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                const uint16_t h = (uint16_t) (u[i / 2] >> (16 * (i & 1)));
+                o[i] = type == WAMX_TYPE_BF16 ? bf16_to_f32(h) : (float) __builtin_bit_cast(_Float16, h);
+            }
+        }
+    }
+}
+template <int V>
+__device__ __forceinline__ void map_store(int32_t type, char * p, const float (&o)[V]) {
+    if constexpr (V == 1) {
+        store_from_f32(p, type, 0, o[0]);
+    } else {
+        uint32_t u[V];
+        if (type == WAMX_TYPE_F32 || type == WAMX_TYPE_I32) {
+#pragma unroll
+            for (int i = 0; i < V; ++i) u[i] = type == WAMX_TYPE_F32 ? __float_as_uint(o[i]) : (uint32_t) (int32_t) o[i];
+#pragma unroll
+            for (int i = 0; i < V / 4; ++i) ((uint4 *) p)[i] = *(uint4 *) &u[4 * i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < V / 2; ++i)
+                u[i] = type == WAMX_TYPE_BF16
+                           ? pack_bf16x2(o[2 * i], o[2 * i + 1])
+                           : (uint32_t) __builtin_bit_cast(uint16_t, (_Float16) o[2 * i]) |
+                                 (uint32_t) __builtin_bit_cast(uint16_t, (_Float16) o[2 * i + 1]) << 16;
+            if constexpr (V == 8) *(uint4 *) p = *(uint4 *) u;
+            else *(uint2 *) p = *(uint2 *) u;
+        }
+    }
+}
+// V elements of one type, bit for bit.
+template <int V>
+__device__ __forceinline__ void map_move(int32_t type, const char * src, char * dst) {
+    const bool wide = type == WAMX_TYPE_F32 || type == WAMX_TYPE_I32;
+    if constexpr (V == 1) {
+        if (wide) *(uint32_t *) dst = *(const uint32_t *) src;
+        else *(uint16_t *) dst = *(const uint16_t *) src;
+    } else if (wide) {
+#pragma unroll
+        for (int i = 0; i < V / 4; ++i) ((uint4 *) dst)[i] = ((const uint4 *) src)[i];
+    } else if constexpr (V == 8) {
+        *(uint4 *) dst = *(const uint4 *) src;
+    } else {
+        *(uint2 *) dst = *(const uint2 *) src;
+    }
+}
+
+template <int OP, int V>
+__global__ __launch_bounds__(256) void map_kernel(MapArgs m) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= m.total) return;
+    uint32_t c[4];
+    const uint32_t q0 = div(i, m.n0), q1 = div(q0, m.n1), q2 = div(q1, m.n2);
+    c[0] = i - q0 * m.n0.d, c[1] = q0 - q1 * m.n1.d, c[2] = q1 - q2 * m.n2.d, c[3] = q2;
+    auto at = [&](const MapOperand & o) {
+        return o.p + c[0] * (V * o.s0) + c[1] * o.s1 + c[2] * o.s2 + c[3] * o.s3;
+    };
+    char * d = at(m.d);
+    if constexpr (OP == kMapConcat) {
+        const uint32_t cd = m.dim == 0 ? c[0] : m.dim == 1 ? c[1] : m.dim == 2 ? c[2] : c[3];
+        // b's pointer is set back by the split, so the coordinates serve both.
+        map_move<V>(m.d.type, cd < m.split ? at(m.a) : at(m.b), d);
+    } else if constexpr (OP == kMapCopy) {
+        if (m.a.type == m.d.type && (V == 1 || m.a.s0 != 0)) {
+            map_move<V>(m.d.type, at(m.a), d);
+        } else {
+            float x[V];
+            map_load<V>(m.a.type, at(m.a), m.a.s0, x);
+            map_store<V>(m.d.type, d, x);
+        }
+    } else {
+        float x[V];
+        map_load<V>(m.a.type, at(m.a), m.a.s0, x);
+        if constexpr (OP == kMapUnary) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) switch (m.uop) {
+                case WAMX_UNARY_GELU: x[e] = gelu_tanh(x[e]); break;
+                case WAMX_UNARY_GELU_ERF: x[e] = gelu_erf(x[e]); break;
+                case WAMX_UNARY_SILU: x[e] = silu(x[e]); break;
+                default: x[e] = x[e] * m.scale + m.bias; break;
+            }
+        } else {
+            float y[V];
+            map_load<V>(m.b.type, at(m.b), m.b.s0, y);
+#pragma unroll
+            for (int e = 0; e < V; ++e) x[e] = OP == kMapAdd ? x[e] + y[e] : x[e] * y[e];
+        }
+        map_store<V>(m.d.type, d, x);
+    }
+}
+
+static int64_t type_bytes(int32_t type) { return type == WAMX_TYPE_F32 || type == WAMX_TYPE_I32 ? 4 : 2; }
+
+// The operand's strides over dst's dims (0 where it has one element); false
+// when a dim repeats by modulo.
+static bool map_operand(const TensorRef & t, const TensorRef & dst, MapOperand & o, int64_t (&st)[4]) {
+    o.p = (char *) t.data;
+    o.type = t.type;
+    for (int i = 0; i < 4; ++i) {
+        if (t.ne[i] != dst.ne[i] && t.ne[i] != 1) return false;
+        st[i] = t.ne[i] == 1 ? 0 : t.nb[i];
+    }
+    return true;
+}
+
+// Runs op over dst's shape; false (nothing launched) when a form is not
+// covered.  concat_dim >= 0: a and b are the parts.
+template <int OP>
+static bool try_map(const TensorRef & a, const TensorRef * b, const TensorRef & dst, int uop, float scale, float bias,
+                    int concat_dim, hipStream_t s) {
+    MapArgs m{};
+    int64_t st[3][4] = {}, ne[4];
+    const int nop = b ? 3 : 2;
+    MapOperand * op[3] = {&m.d, &m.a, &m.b};
+    for (int i = 0; i < 4; ++i) ne[i] = dst.ne[i];
+    m.d = MapOperand{(char *) dst.data, 0, 0, 0, 0, dst.type};
+    for (int i = 0; i < 4; ++i) st[0][i] = dst.nb[i];
+    int64_t split = 0;
+    if (concat_dim >= 0) {
+        for (int k = 1; k < 3; ++k) {
+            const TensorRef & t = k == 1 ? a : *b;
+            op[k]->p = (char *) t.data;
+            op[k]->type = t.type;
+            for (int i = 0; i < 4; ++i) st[k][i] = t.nb[i];
+        }
+        split = a.ne[concat_dim];
+        m.b.p -= split * st[2][concat_dim];
+    } else if (!map_operand(a, dst, m.a, st[1]) || (b && !map_operand(*b, dst, m.b, st[2]))) {
+        return false;
+    }
+    // Merge dims that every operand walks as one; drop dims of one element.
+    int n = 0, cd = -1;
+    int64_t e[4], t[3][4];
+    bool open = false;  // the last kept dim may take the next one in
+    for (int i = 0; i < 4; ++i) {
+        if (ne[i] == 1 && i != concat_dim) continue;
+        bool join = open && i != concat_dim;
+        for (int k = 0; k < nop && join; ++k) join = st[k][i] == t[k][n - 1] * e[n - 1];
+        if (join) {
+            e[n - 1] *= ne[i];
+        } else {
+            e[n] = ne[i];
+            for (int k = 0; k < nop; ++k) t[k][n] = st[k][i];
+            if (i == concat_dim) cd = n;
+            ++n;
+        }
+        open = i != concat_dim;
+    }
+    if (n == 0) {
+        e[0] = 1;
+        for (int k = 0; k < nop; ++k) t[k][0] = type_bytes(op[k]->type);
+        n = 1;
+    }
+    int64_t count = 1;
+    for (int i = 0; i < n; ++i) {
+        if (count > INT32_MAX / std::max<int64_t>(e[i], 1)) return false;
+        count *= e[i];
+    }
+    // Elements per thread: whole chunks of dim 0 at aligned addresses in every
+    // operand; 8 where that still gives two workgroups per CU.
+    auto fits = [&](int v) {
+        if (e[0] % v || (cd == 0 && split % v)) return false;
+        for (int k = 0; k < nop; ++k) {
+            const int64_t es = type_bytes(op[k]->type), al = std::min<int64_t>(16, v * es);
+            if (t[k][0] == 0 && k > 0 && concat_dim < 0) continue;
+            if (t[k][0] != es || (uintptr_t) op[k]->p % (uintptr_t) al) return false;
+            for (int i = 1; i < n; ++i)
+                if (t[k][i] % al) return false;
+        }
+        return true;
+    };
+    const int v = count >= 8 * 256 * 512 && fits(8) ? 8 : fits(4) ? 4 : 1;
+    uint32_t d[4] = {1, 1, 1, 1};
+    for (int i = 0; i < n; ++i) d[i] = (uint32_t) (i == 0 ? e[0] / v : e[i]);
+    m.n0 = fast_div(d[0]), m.n1 = fast_div(d[1]), m.n2 = fast_div(d[2]);
+    for (int k = 0; k < nop; ++k) {
+        op[k]->s0 = t[k][0];
+        op[k]->s1 = n > 1 ? t[k][1] : 0;
+        op[k]->s2 = n > 2 ? t[k][2] : 0;
+        op[k]->s3 = n > 3 ? t[k][3] : 0;
+    }
+    m.total = (uint32_t) (count / v);
+    m.scale = scale, m.bias = bias, m.uop = uop, m.dim = cd;
+    m.split = (uint32_t) (cd == 0 ? split / v : split);
+    const dim3 grid((m.total + 255) / 256);
+    if (v == 8) hipLaunchKernelGGL((map_kernel<OP, 8>), grid, dim3(256), 0, s, m);
+    else if (v == 4) hipLaunchKernelGGL((map_kernel<OP, 4>), grid, dim3(256), 0, s, m);
+    else hipLaunchKernelGGL((map_kernel<OP, 1>), grid, dim3(256), 0, s, m);
+    return true;
 }
 
 // A copy between two same-shape views of 2-byte elements that transposes
@@ -200,16 +457,26 @@ __global__ void get_rows_kernel(Ref4 a, const int32_t * rows, int64_t rows_ld, R
     const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     int64_t i0, i1, i2, i3;
-    unravel(i, dst, i0, i1, i2, i3);
+    if (n <= INT32_MAX) {  // 32-bit divisions
+        const uint32_t n0 = (uint32_t) dst.ne0, n1 = (uint32_t) dst.ne1, n2 = (uint32_t) dst.ne2;
+        const uint32_t q0 = (uint32_t) i / n0, q1 = q0 / n1, q2 = q1 / n2;
+        i0 = (uint32_t) i - q0 * n0, i1 = q0 - q1 * n1, i2 = q1 - q2 * n2, i3 = q2;
+    } else {
+        unravel(i, dst, i0, i1, i2, i3);
+    }
     const int64_t r = rows[i1 + i2 * rows_ld];
     st(dst, at(dst, i0, i1, i2, i3), ld(a, at(a, i0, r, i2 % a.ne2, i3 % a.ne3)));
 }
 
 // SOFT_MAX_EXT: y = exp(w - max) / sum over ne0 with w = scale * x + mask
 // (mask row i1 of plane (i2 % ne2, i3 % ne3); no mask when m.data is null).
-// One workgroup per row.
-__global__ __launch_bounds__(256) void softmax_kernel(Ref4 x, Ref4 m, Ref4 y, float scale) {
+// One workgroup of W waves per row.  PER > 0: the row's values stay in
+// registers (PER per thread), so it is read and written once; 0: any length.
+// W = 1 for rows of at most 64, where three of four waves would hold nothing.
+template <int PER, int W>
+__global__ __launch_bounds__(64 * W) void softmax_kernel(Ref4 x, Ref4 m, Ref4 y, float scale) {
     __shared__ float red[4];
+    constexpr int T = 64 * W;
     const int64_t row = blockIdx.x;
     const int64_t r1 = row % x.ne1, r2 = (row / x.ne1) % x.ne2, r3 = row / (x.ne1 * x.ne2);
     const char * xr = at(x, 0, r1, r2, r3);
@@ -219,22 +486,49 @@ __global__ __launch_bounds__(256) void softmax_kernel(Ref4 x, Ref4 m, Ref4 y, fl
         const float v = *(const float *) (xr + c * x.nb0) * scale;
         return mr ? v + ld(m, mr + c * m.nb0) : v;
     };
+    constexpr int R = PER > 0 ? PER : 1;
+    float v[R];
     float mx = -INFINITY;
-    for (int64_t c = threadIdx.x; c < x.ne0; c += 256) mx = fmaxf(mx, w_at(c));
-    mx = wave_max(mx);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    float sum = 0.0f;
-    for (int64_t c = threadIdx.x; c < x.ne0; c += 256) {
-        const float e = expf(w_at(c) - mx);
-        *(float *) (yr + c * y.nb0) = e;
-        sum += e;
+    if constexpr (PER > 0) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) v[i] = w_at(min((int64_t) threadIdx.x + i * T, x.ne0 - 1));
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if ((int64_t) threadIdx.x + i * T < x.ne0) mx = fmaxf(mx, v[i]);
+    } else {
+        for (int64_t c = threadIdx.x; c < x.ne0; c += T) mx = fmaxf(mx, w_at(c));
     }
-    sum = block_sum(sum, red);
+    mx = wave_max(mx);
+    if constexpr (W > 1) {
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+        __syncthreads();
+        mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    }
+    float sum = 0.0f;
+    if constexpr (PER > 0) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            v[i] = expf(v[i] - mx);
+            if ((int64_t) threadIdx.x + i * T < x.ne0) sum += v[i];
+        }
+    } else {
+        for (int64_t c = threadIdx.x; c < x.ne0; c += T) {
+            const float e = expf(w_at(c) - mx);
+            *(float *) (yr + c * y.nb0) = e;
+            sum += e;
+        }
+    }
+    sum = W > 1 ? block_sum(sum, red) : wave_sum(sum);
     const float inv = 1.0f / sum;
-    for (int64_t c = threadIdx.x; c < x.ne0; c += 256) *(float *) (yr + c * y.nb0) *= inv;
+    if constexpr (PER > 0) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const int64_t c = (int64_t) threadIdx.x + i * T;
+            if (c < x.ne0) *(float *) (yr + c * y.nb0) = v[i] * inv;
+        }
+    } else {
+        for (int64_t c = threadIdx.x; c < x.ne0; c += T) *(float *) (yr + c * y.nb0) *= inv;
+    }
 }
 
 // ROPE mode NORMAL on [head_dim, heads, tokens(, ne3)]: pairs (2i, 2i+1) for
@@ -243,11 +537,18 @@ __global__ void rope_kernel(Ref4 x, const int32_t * pos, Ref4 y, int n_dims, flo
     const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= npairs) return;
     const int64_t half = (x.ne0 + 1) / 2;
-    const int64_t ip = i % half;
-    int64_t rest = i / half;
-    const int64_t i1 = rest % x.ne1;
-    rest /= x.ne1;
-    const int64_t i2 = rest % x.ne2, i3 = rest / x.ne2;
+    int64_t ip, i1, i2, i3;
+    if (npairs <= INT32_MAX) {  // 32-bit divisions
+        const uint32_t h = (uint32_t) half, n1 = (uint32_t) x.ne1, n2 = (uint32_t) x.ne2;
+        const uint32_t q0 = (uint32_t) i / h, q1 = q0 / n1, q2 = q1 / n2;
+        ip = (uint32_t) i - q0 * h, i1 = q0 - q1 * n1, i2 = q1 - q2 * n2, i3 = q2;
+    } else {
+        ip = i % half;
+        int64_t rest = i / half;
+        i1 = rest % x.ne1;
+        rest /= x.ne1;
+        i2 = rest % x.ne2, i3 = rest / x.ne2;
+    }
     const int64_t e = 2 * ip;
     const char * px = at(x, e, i1, i2, i3);
     char * py = at(y, e, i1, i2, i3);
@@ -477,6 +778,15 @@ __global__ void fill_f32_kernel(float * dst, int64_t n, float v) {
 static int64_t nel(const TensorRef & t) { return t.ne[0] * t.ne[1] * t.ne[2] * t.ne[3]; }
 static dim3 grid1d(int64_t n) { return dim3((unsigned) ((n + 255) / 256)); }
 
+static bool dense(const TensorRef & t) {
+    int64_t b = type_bytes(t.type);
+    for (int i = 0; i < 4; ++i) {
+        if (t.ne[i] != 1 && t.nb[i] != b) return false;
+        b *= t.ne[i];
+    }
+    return true;
+}
+
 hipError_t launch_copy(const TensorRef & src, const TensorRef & dst, hipStream_t s) {
     const int64_t n = nel(dst);
     if (n <= 0) return hipSuccess;
@@ -503,6 +813,15 @@ hipError_t launch_copy(const TensorRef & src, const TensorRef & dst, hipStream_t
             hipLaunchKernelGGL(transpose01_kernel, grid, dim3(256), 0, s, to_ref4(src), to_ref4(dst));
         return hipGetLastError();
     }
+    if (same_shape && try_map<kMapCopy>(src, nullptr, dst, 0, 0, 0, -1, s)) return hipGetLastError();
+    if (!same_shape && dense(src) && dense(dst)) {  // a reshape: both in memory order
+        TensorRef f = src, d = dst;
+        for (TensorRef * t : {&f, &d}) {
+            t->ne[0] = n;
+            t->ne[1] = t->ne[2] = t->ne[3] = 1;
+        }
+        if (try_map<kMapCopy>(f, nullptr, d, 0, 0, 0, -1, s)) return hipGetLastError();
+    }
     hipLaunchKernelGGL(copy_kernel, grid1d(n), dim3(256), 0, s, to_ref4(src), to_ref4(dst), n);
     return hipGetLastError();
 }
@@ -510,6 +829,10 @@ hipError_t launch_copy(const TensorRef & src, const TensorRef & dst, hipStream_t
 hipError_t launch_binary(int op, const TensorRef & a, const TensorRef & b, const TensorRef & dst, hipStream_t s) {
     const int64_t n = nel(dst);
     if (n <= 0) return hipSuccess;
+    if (op == 0 ? try_map<kMapAdd>(a, &b, dst, 0, 0, 0, -1, s)
+        : op == 1 ? try_map<kMapMul>(a, &b, dst, 0, 0, 0, -1, s)
+                  : try_map<kMapCopy>(b, nullptr, dst, 0, 0, 0, -1, s))
+        return hipGetLastError();
     hipLaunchKernelGGL(binary_kernel, grid1d(n), dim3(256), 0, s, op, to_ref4(a), to_ref4(b), to_ref4(dst), n);
     return hipGetLastError();
 }
@@ -517,6 +840,7 @@ hipError_t launch_binary(int op, const TensorRef & a, const TensorRef & b, const
 hipError_t launch_unary(int op, const TensorRef & a, const TensorRef & dst, float scale, float bias, hipStream_t s) {
     const int64_t n = nel(dst);
     if (n <= 0) return hipSuccess;
+    if (try_map<kMapUnary>(a, nullptr, dst, op, scale, bias, -1, s)) return hipGetLastError();
     hipLaunchKernelGGL(unary_kernel, grid1d(n), dim3(256), 0, s, op, to_ref4(a), to_ref4(dst), scale, bias, n);
     return hipGetLastError();
 }
@@ -524,6 +848,7 @@ hipError_t launch_unary(int op, const TensorRef & a, const TensorRef & dst, floa
 hipError_t launch_concat(const TensorRef & a, const TensorRef & b, const TensorRef & dst, int dim, hipStream_t s) {
     const int64_t n = nel(dst);
     if (n <= 0) return hipSuccess;
+    if (try_map<kMapConcat>(a, &b, dst, 0, 0, 0, dim, s)) return hipGetLastError();
     hipLaunchKernelGGL(concat_kernel, grid1d(n), dim3(256), 0, s, to_ref4(a), to_ref4(b), to_ref4(dst), dim, n);
     return hipGetLastError();
 }
@@ -539,8 +864,15 @@ hipError_t launch_softmax_f32(const TensorRef & x, const TensorRef & mask, const
                               hipStream_t s) {
     const int64_t rows = x.ne[1] * x.ne[2] * x.ne[3];
     if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(softmax_kernel, dim3((unsigned) rows), dim3(256), 0, s, to_ref4(x), to_ref4(mask), to_ref4(y),
-                       scale);
+#define WAMX_SOFTMAX(PER, W)                                                                                       \
+    hipLaunchKernelGGL((softmax_kernel<PER, W>), dim3((unsigned) rows), dim3(64 * W), 0, s, to_ref4(x), to_ref4(mask), \
+                       to_ref4(y), scale)
+    if (x.ne[0] <= 64) WAMX_SOFTMAX(1, 1);
+    else if (x.ne[0] <= 512) WAMX_SOFTMAX(2, 4);
+    else if (x.ne[0] <= 2048) WAMX_SOFTMAX(8, 4);
+    else if (x.ne[0] <= 4096) WAMX_SOFTMAX(16, 4);
+    else WAMX_SOFTMAX(0, 4);
+#undef WAMX_SOFTMAX
     return hipGetLastError();
 }
 

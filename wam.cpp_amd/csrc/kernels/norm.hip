@@ -80,6 +80,10 @@ __global__ __launch_bounds__(kNormThreads) void norm_mod_bf16_kernel(const uint1
     for (int c = threadIdx.x + kMaxCache * kNormThreads; c < cols; c += kNormThreads) emit(c, bf16_to_f32(xr[c]));
 }
 
+// CACHE: elements per thread held in registers, all loaded before the first
+// use, so a row up to CACHE x 256 columns costs one memory round trip; longer
+// rows read the rest again.
+template <int CACHE>
 __global__ __launch_bounds__(kNormThreads) void rms_norm_bf16_f32_kernel(const uint16_t * __restrict__ x, int64_t ldx,
                                                                           const uint16_t * __restrict__ w,
                                                                           float * __restrict__ y, int64_t ldy, int cols,
@@ -87,32 +91,39 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_bf16_f32_kernel(const u
     __shared__ float red[kNormThreads / 64];
     const int64_t row = blockIdx.x;
     const uint16_t * xr = x + row * ldx;
-    float v[kMaxCache];
+    uint16_t h[CACHE], wh[CACHE];
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i) {
+        const int c = min((int) threadIdx.x + i * kNormThreads, cols - 1);
+        h[i] = xr[c];
+        wh[i] = w[c];
+    }
+    float v[CACHE];
     float sum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < kMaxCache; ++i) {
-        const int c = threadIdx.x + i * kNormThreads;
-        v[i] = c < cols ? bf16_to_f32(xr[c]) : 0.0f;
+    for (int i = 0; i < CACHE; ++i) {
+        v[i] = (int) threadIdx.x + i * kNormThreads < cols ? bf16_to_f32(h[i]) : 0.0f;
         sum = fmaf(v[i], v[i], sum);
     }
-    for (int c = threadIdx.x + kMaxCache * kNormThreads; c < cols; c += kNormThreads) {
+    for (int c = threadIdx.x + CACHE * kNormThreads; c < cols; c += kNormThreads) {
         const float t = bf16_to_f32(xr[c]);
         sum = fmaf(t, t, sum);
     }
     const float inv_rms = rsqrtf(block_sum(sum, red) / (float) cols + eps);
     float * yr = y + row * ldy;
 #pragma unroll
-    for (int i = 0; i < kMaxCache; ++i) {
+    for (int i = 0; i < CACHE; ++i) {
         const int c = threadIdx.x + i * kNormThreads;
-        if (c < cols) yr[c] = v[i] * inv_rms * bf16_to_f32(w[c]);
+        if (c < cols) yr[c] = v[i] * inv_rms * bf16_to_f32(wh[i]);
     }
-    for (int c = threadIdx.x + kMaxCache * kNormThreads; c < cols; c += kNormThreads)
+    for (int c = threadIdx.x + CACHE * kNormThreads; c < cols; c += kNormThreads)
         yr[c] = bf16_to_f32(xr[c]) * inv_rms * bf16_to_f32(w[c]);
 }
 
 // p7-fusions.patch:19-51: one-pass E[x], E[x^2]; out = (n + n*scale) + shift,
 // each product and sum rounded separately (no contraction).
 #pragma clang fp contract(off)
+template <int CACHE>
 __global__ __launch_bounds__(kNormThreads) void norm_mod_f32_kernel(const float * __restrict__ x, int64_t ldx,
                                                                      const float * __restrict__ scale,
                                                                      const float * __restrict__ shift, int64_t ss,
@@ -120,48 +131,81 @@ __global__ __launch_bounds__(kNormThreads) void norm_mod_f32_kernel(const float 
     __shared__ float red[kNormThreads / 64];
     const int64_t row = blockIdx.x;
     const float * xr = x + row * ldx;
+    const float * sc = scale + row * ss;
+    const float * sh = shift + row * ss;
+    float v[CACHE], vs[CACHE], vh[CACHE];
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i) {
+        const int c = min((int) threadIdx.x + i * kNormThreads, cols - 1);
+        v[i] = xr[c];
+        vs[i] = sc[c];
+        vh[i] = sh[c];
+    }
     float s1 = 0.0f, s2 = 0.0f;
-    for (int c = threadIdx.x; c < cols; c += kNormThreads) {
-        const float xi = xr[c];
+    auto add = [&](float xi) {
         s1 += xi;
         s2 += xi * xi;
-    }
+    };
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i)
+        if ((int) threadIdx.x + i * kNormThreads < cols) add(v[i]);
+    for (int c = threadIdx.x + CACHE * kNormThreads; c < cols; c += kNormThreads) add(xr[c]);
     s1 = block_sum(s1, red);
     s2 = block_sum(s2, red);
     const float mean = s1 / (float) cols;
     const float var = s2 / (float) cols - mean * mean;
     const float inv_std = rsqrtf(var + eps);
-    const float * sc = scale + row * ss;
-    const float * sh = shift + row * ss;
     float * yr = y + row * (int64_t) cols;
-    for (int c = threadIdx.x; c < cols; c += kNormThreads) {
-        const float n = (xr[c] - mean) * inv_std;
-        const float scaled = n * sc[c];
-        yr[c] = (n + scaled) + sh[c];
+    auto emit = [&](int c, float xi, float a, float b) {
+        const float n = (xi - mean) * inv_std;
+        const float scaled = n * a;
+        yr[c] = (n + scaled) + b;
+    };
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i) {
+        const int c = threadIdx.x + i * kNormThreads;
+        if (c < cols) emit(c, v[i], vs[i], vh[i]);
     }
+    for (int c = threadIdx.x + CACHE * kNormThreads; c < cols; c += kNormThreads) emit(c, xr[c], sc[c], sh[c]);
 }
 
 // ggml NORM / RMS_NORM on f32 rows (stock ggml ops of the F32 profile).
+template <int CACHE>
 __global__ __launch_bounds__(kNormThreads) void norm_f32_kernel(const float * __restrict__ x, int64_t ldx,
                                                                  float * __restrict__ y, int64_t ldy, int cols,
                                                                  float eps, int rms) {
     __shared__ float red[kNormThreads / 64];
     const int64_t row = blockIdx.x;
     const float * xr = x + row * ldx;
+    float v[CACHE];
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i) v[i] = xr[min((int) threadIdx.x + i * kNormThreads, cols - 1)];
     float mean = 0.0f;
     if (!rms) {
         float s = 0.0f;
-        for (int c = threadIdx.x; c < cols; c += kNormThreads) s += xr[c];
+#pragma unroll
+        for (int i = 0; i < CACHE; ++i)
+            if ((int) threadIdx.x + i * kNormThreads < cols) s += v[i];
+        for (int c = threadIdx.x + CACHE * kNormThreads; c < cols; c += kNormThreads) s += xr[c];
         mean = block_sum(s, red) / (float) cols;
     }
     float s2 = 0.0f;
-    for (int c = threadIdx.x; c < cols; c += kNormThreads) {
-        const float d = xr[c] - mean;
+    auto add = [&](float xi) {
+        const float d = xi - mean;
         s2 += d * d;
-    }
+    };
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i)
+        if ((int) threadIdx.x + i * kNormThreads < cols) add(v[i]);
+    for (int c = threadIdx.x + CACHE * kNormThreads; c < cols; c += kNormThreads) add(xr[c]);
     const float inv = rsqrtf(block_sum(s2, red) / (float) cols + eps);
     float * yr = y + row * ldy;
-    for (int c = threadIdx.x; c < cols; c += kNormThreads) yr[c] = (xr[c] - mean) * inv;
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i) {
+        const int c = threadIdx.x + i * kNormThreads;
+        if (c < cols) yr[c] = (v[i] - mean) * inv;
+    }
+    for (int c = threadIdx.x + CACHE * kNormThreads; c < cols; c += kNormThreads) yr[c] = (xr[c] - mean) * inv;
 }
 
 __global__ void gated_residual_f32_kernel(const float * __restrict__ r, int64_t ldr, const float * __restrict__ b,
@@ -193,6 +237,19 @@ __global__ void bias_gelu_bf16_kernel(const uint16_t * __restrict__ x, const uin
     if (i >= n) return;
     const float v = bf16_to_f32(x[i]) + bf16_to_f32(bias[i % width]);
     y[i] = f32_to_bf16(gelu_tanh(v));
+}
+
+// The same for 16-byte aligned rows of a multiple of 8 columns, 8 per thread.
+__global__ __launch_bounds__(256) void bias_gelu_bf16_vec(const uint4 * __restrict__ x, const uint4 * __restrict__ bias,
+                                                          uint4 * __restrict__ y, uint32_t n, uint32_t width) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    float v[8], b[8];
+    unpack8(x[i], v);
+    unpack8(bias[i % width], b);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = gelu_tanh(v[e] + b[e]);
+    y[i] = pack8(v);
 }
 
 // ---------------------------------------------------------------------------
@@ -309,25 +366,37 @@ hipError_t launch_norm_mod_bf16(const void * x, int64_t ldx, const void * scale,
 
 hipError_t launch_rms_norm_bf16_f32(const void * x, int64_t ldx, const void * w, float * y, int64_t ldy, int64_t rows,
                                     int64_t cols, float eps, hipStream_t s) {
-    if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(rms_norm_bf16_f32_kernel, dim3((unsigned) rows), dim3(kNormThreads), 0, s, (const uint16_t *) x,
-                       ldx, (const uint16_t *) w, y, ldy, (int) cols, eps);
+    if (rows <= 0 || cols <= 0) return hipSuccess;
+    const dim3 grid((unsigned) rows), block(kNormThreads);
+    const uint16_t * xh = (const uint16_t *) x, * wh = (const uint16_t *) w;
+    if (cols <= 4 * kNormThreads)
+        hipLaunchKernelGGL(rms_norm_bf16_f32_kernel<4>, grid, block, 0, s, xh, ldx, wh, y, ldy, (int) cols, eps);
+    else if (cols <= 12 * kNormThreads)
+        hipLaunchKernelGGL(rms_norm_bf16_f32_kernel<12>, grid, block, 0, s, xh, ldx, wh, y, ldy, (int) cols, eps);
+    else
+        hipLaunchKernelGGL(rms_norm_bf16_f32_kernel<16>, grid, block, 0, s, xh, ldx, wh, y, ldy, (int) cols, eps);
     return hipGetLastError();
 }
 
 hipError_t launch_norm_mod_f32(const float * x, int64_t ldx, const float * scale, const float * shift, int64_t ss,
                                float * y, int64_t rows, int64_t cols, float eps, hipStream_t s) {
-    if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(norm_mod_f32_kernel, dim3((unsigned) rows), dim3(kNormThreads), 0, s, x, ldx, scale, shift, ss, y,
-                       (int) cols, eps);
+    if (rows <= 0 || cols <= 0) return hipSuccess;
+    const dim3 grid((unsigned) rows), block(kNormThreads);
+    if (cols <= 4 * kNormThreads)
+        hipLaunchKernelGGL(norm_mod_f32_kernel<4>, grid, block, 0, s, x, ldx, scale, shift, ss, y, (int) cols, eps);
+    else
+        hipLaunchKernelGGL(norm_mod_f32_kernel<12>, grid, block, 0, s, x, ldx, scale, shift, ss, y, (int) cols, eps);
     return hipGetLastError();
 }
 
 hipError_t launch_norm_f32(const float * x, int64_t ldx, float * y, int64_t ldy, int64_t rows, int64_t cols, float eps,
                            bool rms, hipStream_t s) {
-    if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(norm_f32_kernel, dim3((unsigned) rows), dim3(kNormThreads), 0, s, x, ldx, y, ldy, (int) cols, eps,
-                       rms ? 1 : 0);
+    if (rows <= 0 || cols <= 0) return hipSuccess;
+    const dim3 grid((unsigned) rows), block(kNormThreads);
+    if (cols <= 4 * kNormThreads)
+        hipLaunchKernelGGL(norm_f32_kernel<4>, grid, block, 0, s, x, ldx, y, ldy, (int) cols, eps, rms ? 1 : 0);
+    else
+        hipLaunchKernelGGL(norm_f32_kernel<16>, grid, block, 0, s, x, ldx, y, ldy, (int) cols, eps, rms ? 1 : 0);
     return hipGetLastError();
 }
 
@@ -354,6 +423,12 @@ hipError_t launch_gated_residual_f32(const float * r, int64_t ldr, const float *
 
 hipError_t launch_bias_gelu_bf16(const void * x, const void * bias, void * y, int64_t n, int64_t width, hipStream_t s) {
     if (n <= 0) return hipSuccess;
+    if (width % 8 == 0 && n / 8 <= INT32_MAX && aligned16(x) && aligned16(bias) && aligned16(y)) {
+        hipLaunchKernelGGL(bias_gelu_bf16_vec, dim3((unsigned) ((n / 8 + 255) / 256)), dim3(256), 0, s,
+                           (const uint4 *) x, (const uint4 *) bias, (uint4 *) y, (uint32_t) (n / 8),
+                           (uint32_t) (width / 8));
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(bias_gelu_bf16_kernel, dim3((unsigned) ((n + 255) / 256)), dim3(256), 0, s, (const uint16_t *) x,
                        (const uint16_t *) bias, (uint16_t *) y, n, width);
     return hipGetLastError();
