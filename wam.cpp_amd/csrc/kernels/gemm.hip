@@ -12,8 +12,9 @@
 //  * gemm_skinny — N <= 64 tokens (the 48-token action expert): HBM-bound
 //                  weight streaming with MFMA 16x16x32, K split across the
 //                  waves of a workgroup and reduced in LDS.
-//  * gemm_f32    — f32 weights (the f32 reference profile, generic MUL_MAT),
-//                  f32 MFMA 16x16x4.
+//  * gemm_gen    — f32 weights (the f32 reference profile, generic MUL_MAT) on
+//                  f32 MFMA 16x16x4, and the few-token bf16 products in
+//                  batches or with unaligned rows.
 #include "../internal.h"
 #include "device.h"
 #include "rowops.h"
@@ -1765,104 +1766,145 @@ static hipError_t run_skinny(const GemmParams & p, bool xf32, bool tiled, void *
 }
 
 // ---------------------------------------------------------------------------
-// gemm_f32: f32 weights (the f32 reference profile, MUL_MAT of two f32
-// tensors, f32 convolutions), products and sums in f32 on MFMA 16x16x4.
+// gemm_gen: the products the LDS-DMA and skinny kernels do not take: f32
+// weights at any size (the f32 reference profile, MUL_MAT of two f32 tensors,
+// f32 convolutions; products and sums in f32 on MFMA 16x16x4), and bf16
+// weights at up to 64 tokens in batches or with rows of any alignment
+// (attention of separate ggml nodes; MFMA 16x16x32).
 //
-// The f32 matrix rate is 1/16 of bf16's (154 TFLOP/s measured on a large
-// product), so the tile needs little LDS bandwidth and the work is bound by
-// the MFMAs at 48 or more tokens and by the weight stream below that.  A
-// workgroup of 4 waves multiplies 16 NT tokens by 64 RG features; K steps of
-// 32 go through two LDS stages with the next step's loads held in registers
-// meanwhile.  In a step, lane group g's 16-byte fragment covers columns 16 q +
-// 4 g .. + 4 of both operands and feeds 4 MFMAs, one column of each group per
-// MFMA (both operands take the same K order, so any order is a valid one).
-// Rows are padded by 4 floats: 16 rows' 16-byte reads cover all 64 banks.
-// K slices (blockIdx.y) write f32 partials that gemm_skinny_reduce sums in
-// slice order.
-// One thread per output with a serial K loop, which this replaced, took
-// 1998 us for 3072 x 48 x 3072 and 9287 us for 14336 x 48 x 3072; now 27 and
-// 67 us (1.4 and 2.6 TB/s of weights), and its error against 64-bit sums over
-// an action layer is a third of the serial sum's.
-// VEC: rows start at 16-byte multiples and K % 4 == 0; else scalar loads of
-// 32 consecutive columns per half wave.
+// A workgroup of 4 waves multiplies 16 NT tokens by 64 RG features.  A K step
+// is 128 bytes of each weight row (32 f32 or 64 bf16), through two LDS stages
+// with the next step's loads held in registers meanwhile.  Lane group g's
+// 16-byte fragments cover bytes 64 q + 16 g .. + 16 of both operands; in f32
+// one feeds 4 MFMAs, one column of each group per MFMA (both operands take the
+// same K order, so any order is a valid one).  Rows are padded by 16 bytes: 16
+// rows' 16-byte reads cover all 64 banks.  Global loads are 16 bytes at the
+// element's own alignment, which gfx950 takes (an odd number of keys makes
+// every other V^T row odd).  K slices (blockIdx.y) write f32 partials that
+// gemm_skinny_reduce sums in slice order.
+//
+// f32 is bound by the MFMAs at 48 or more tokens (1/16 of the bf16 rate: 154
+// TFLOP/s measured on a large product) and by the weight stream below that.
+// One thread per output with a serial K loop took 1998 us for 3072 x 48 x 3072
+// and 9287 us for 14336 x 48 x 3072; now 27 and 67 us (1.4 and 2.6 TB/s of
+// weights), and the error against 64-bit sums over an action layer is a third
+// of the serial sum's.  The 128 x 128 tiles took 258 us for a head's 128 x 48
+// x 3121 product of probabilities and V^T in 24 heads; now 13.6 and 4.9 us of reduce
+// (10 slices).
 // ---------------------------------------------------------------------------
-constexpr int kF32BK = 32, kF32Pitch = kF32BK + 4, kF32Threads = 256;
+constexpr int kGenThreads = 256;
+constexpr int kGenPitch = 128 + 16;  // bytes per LDS row
 
-template <int NT, int RG, bool VEC, bool XBF>
-__global__ __launch_bounds__(kF32Threads) void gemm_f32(GemmParams p, float * part, int nt_m, int nt_n, int ks) {
+struct __attribute__((packed, aligned(2))) loose16 {
+    uint32_t x, y, z, w;
+};
+struct __attribute__((packed, aligned(2))) loose8 {
+    uint32_t x, y;
+};
+__device__ __forceinline__ uint4 load_loose16(const char * p) {
+    const loose16 v = *(const loose16 *) p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+// WBF: bf16 weights, else f32.  XC: activations of the other type, rounded to
+// bf16 or widened on their way into LDS.
+template <int NT, int RG, bool WBF, bool XC>
+__global__ __launch_bounds__(kGenThreads, 2) void gemm_gen(GemmParams p, float * part, int nt_m, int nt_n, int ks) {
     constexpr int BM = 16 * NT, BN = 64 * RG, ROWS = BM + BN;
-    constexpr int PER = ROWS * kF32BK / 4 / kF32Threads;  // 16-byte chunks per thread per step
-    constexpr int RPC = kF32Threads / 8;                  // rows per chunk instruction
-    constexpr int LEFT = ROWS - PER * RPC;                // rows of a last part-full instruction
-    constexpr int NL = PER + (LEFT > 0);
-    static_assert(!(VEC && XBF), "bf16 activations take the scalar loads");
-    __shared__ __align__(16) float st[2][ROWS * kF32Pitch];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int EPC = WBF ? 8 : 4, BK = 8 * EPC;        // elements per 16-byte chunk, per step
+    constexpr int WS = WBF ? 2 : 4, XS = XC ? 6 - WS : WS;  // element sizes
+    constexpr int NL = (ROWS + 31) / 32;                   // 32 rows of 8 chunks per load instruction
+    constexpr int NX = XC && WBF ? (BM + 31) / 32 : 1;     // second halves of f32 activations
+    __shared__ __align__(16) char st[2][ROWS * kGenPitch];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, r16 = lane & 15;
     const int64_t b2 = blockIdx.z % p.B2, b3 = blockIdx.z / p.B2;
-    const float * w = (const float *) p.w + (b2 / p.r2) * p.w_bs2 + (b3 / p.r3) * p.w_bs3;
-    const char * x = (const char *) p.x + (b2 * p.x_bs2 + b3 * p.x_bs3) * (XBF ? 2 : 4);
     int tm, tn;
     tile_coords((int) blockIdx.x, nt_m, nt_n, tm, tn);
-    const int64_t n0 = (int64_t) tn * BM, m0 = (int64_t) tm * BN;
-    const int64_t kb = (int64_t) blockIdx.y * ks;
+    const int64_t n0 = (int64_t) tn * BM, m0 = (int64_t) tm * BN, kb = (int64_t) blockIdx.y * ks;
+    const char * xt = (const char *) p.x + (b2 * p.x_bs2 + b3 * p.x_bs3 + n0 * p.ldx + kb) * XS;
+    const char * wt = (const char *) p.w + ((b2 / p.r2) * p.w_bs2 + (b3 / p.r3) * p.w_bs3 + m0 * p.ldw + kb) * WS;
     const int klen = (int) min(p.K - kb, (int64_t) ks);
-    const int nsteps = (klen + kF32BK - 1) / kF32BK;
-
-    // A load instruction takes 32 rows (VEC: 8 threads of 4 columns a row) or 8
-    // (32 threads of one column a row).
-    float4 rv[VEC ? NL : 1];
-    float rs[VEC ? 1 : 4 * NL];
-    // Sources are byte offsets from the tile's first token and weight row,
-    // so a step adds one offset to each.
-    const char * xt = x + (n0 * p.ldx + kb) * (XBF ? 2 : 4);
-    const char * wt = (const char *) (w + m0 * p.ldw + kb);
-    constexpr int RPI = VEC ? RPC : RPC / 4, NI = VEC ? NL : 4 * NL;
-    const int64_t ldx = p.ldx, ldw = p.ldw;
+    const int nsteps = (klen + BK - 1) / BK;
     const int nlast = (int) min(p.N - n0, (int64_t) BM) - 1, mlast = (int) min(p.M - m0, (int64_t) BN) - 1;
-    const char * src[NI];
+
+    // Row pointers at the thread's chunk; a wave's 8 rows of an instruction are
+    // all tokens or all weights (BM % 8 == 0).
+    const char * src[NL];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-        const int r = min(i * RPI + tid / (VEC ? 8 : 32), ROWS - 1);
-        const char * xr = xt + (int64_t) min(r, nlast) * ldx * (XBF ? 2 : 4);
-        const char * wr = wt + (int64_t) min(max(r - BM, 0), mlast) * ldw * 4;
-        src[i] = r < BM ? xr : wr;
+    for (int i = 0; i < NL; ++i) {
+        const int r = i * 32 + (tid >> 3);
+        const char * xr = xt + ((int64_t) min(r, nlast) * p.ldx + EPC * (tid & 7)) * XS;
+        const char * wr = wt + ((int64_t) min(max(r - BM, 0), mlast) * p.ldw + EPC * (tid & 7)) * WS;
+        src[i] = i * 32 + wave * 8 < BM ? xr : wr;
     }
+    // A chunk that would reach past the slice is loaded further left, to end
+    // with it, and shifted into place on its way into LDS (columns left of the
+    // slice are the row's own: K >= EPC).
+    const int cb = EPC * (tid & 7);  // the chunk's first column in a step
+    uint4 raw[NL], raw2[NX];
     auto load = [&](int step) {
-        if constexpr (VEC) {
-            const int k = step * kF32BK + 4 * (tid & 7), kc = min(k, klen - 4);
+        if (p.K < EPC) return;
+        const int64_t k = min(step * BK + cb, klen - EPC) - cb;
 #pragma unroll
-            for (int i = 0; i < NL; ++i) {
-                rv[i] = *(const float4 *) (src[i] + (int64_t) kc * 4);
-            }
-        } else {
-            const int k = step * kF32BK + (tid & 31), kc = min(k, klen - 1);
-#pragma unroll
-            for (int i = 0; i < 4 * NL; ++i) {
-                // BM is a multiple of the rows of an instruction: all of them tokens, or all weights.
-                if (XBF && i * RPI < BM) rs[i] = bf16_to_f32(*(const uint16_t *) (src[i] + (int64_t) kc * 2));
-                else rs[i] = *(const float *) (src[i] + (int64_t) kc * 4);
+        for (int i = 0; i < NL; ++i) {
+            if (XC && i * 32 + wave * 8 < BM) {
+                if constexpr (WBF) {
+                    raw[i] = load_loose16(src[i] + k * 4);
+                    raw2[i < NX ? i : 0] = load_loose16(src[i] + k * 4 + 16);
+                } else {
+                    const loose8 v = *(const loose8 *) (src[i] + k * 2);
+                    raw[i] = make_uint4(v.x, v.y, 0, 0);
+                }
+            } else {
+                raw[i] = load_loose16(src[i] + k * WS);
             }
         }
     };
-    // The K tail is zeroed here and not at the load: a use of a loaded register
-    // right after its load would make the wave wait for it before the MFMAs.
-    auto store = [&](int step, float * s) {
-        if constexpr (VEC) {
-            const bool ok = step * kF32BK + 4 * (tid & 7) < klen;
-#pragma unroll
-            for (int i = 0; i < NL; ++i) {
-                const int r = i * RPC + (tid >> 3);
-                if (i < PER || r < ROWS)
-                    *(float4 *) (s + r * kF32Pitch + 4 * (tid & 7)) = ok ? rv[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    auto store = [&](int step, char * s) {
+        if (p.K < EPC) {  // a few columns in all: element by element
+#pragma unroll 1
+            for (int i = tid; i < ROWS * BK; i += kGenThreads) {
+                const int r = i / BK, c = i % BK;
+                uint32_t v = 0;
+                if (c < klen && r < BM) {
+                    const char * q = xt + ((int64_t) min(r, nlast) * p.ldx + c) * XS;
+                    if (XS == 4) v = WBF ? f32_to_bf16(*(const float *) q) : *(const uint32_t *) q;
+                    else v = (uint32_t) *(const uint16_t *) q << (WBF ? 0 : 16);
+                } else if (c < klen) {
+                    const char * q = wt + ((int64_t) min(r - BM, mlast) * p.ldw + c) * WS;
+                    v = WBF ? *(const uint16_t *) q : *(const uint32_t *) q;
+                }
+                if (WBF) *(uint16_t *) (s + r * kGenPitch + 2 * c) = (uint16_t) v;
+                else *(uint32_t *) (s + r * kGenPitch + 4 * c) = v;
             }
-        } else {
-            const bool ok = step * kF32BK + (tid & 31) < klen;
+            return;
+        }
+        const int d = max(step * BK + cb - (klen - EPC), 0);  // elements to shift out
 #pragma unroll
-            for (int i = 0; i < 4 * NL; ++i) {
-                const int r = i * (RPC / 4) + (tid >> 5);
-                if (i < 4 * PER || r < ROWS) s[r * kF32Pitch + (tid & 31)] = ok ? rs[i] : 0.0f;
+        for (int i = 0; i < NL; ++i) {
+            const int r = i * 32 + (tid >> 3);
+            uint4 v = raw[i];
+            if (XC && i * 32 + wave * 8 < BM) {
+                if constexpr (WBF) {
+                    const uint4 u = raw2[i < NX ? i : 0];
+                    v = make_uint4(pack_bf16x2(__uint_as_float(v.x), __uint_as_float(v.y)),
+                                   pack_bf16x2(__uint_as_float(v.z), __uint_as_float(v.w)),
+                                   pack_bf16x2(__uint_as_float(u.x), __uint_as_float(u.y)),
+                                   pack_bf16x2(__uint_as_float(u.z), __uint_as_float(u.w)));
+                } else {
+                    v = make_uint4(v.x << 16, v.x & 0xFFFF0000u, v.y << 16, v.y & 0xFFFF0000u);
+                }
             }
+            if (step * BK + BK > klen) {
+                const int dw = d * WS / 4;
+                if (dw & 1) v = make_uint4(v.y, v.z, v.w, 0);
+                if (dw & 2) v = make_uint4(v.z, v.w, 0, 0);
+                if (WBF && (d & 1))
+                    v = make_uint4(v.x >> 16 | v.y << 16, v.y >> 16 | v.z << 16, v.z >> 16 | v.w << 16, v.w >> 16);
+                if (d >= EPC) v = make_uint4(0, 0, 0, 0);
+            }
+            if ((i + 1) * 32 <= ROWS || r < ROWS) *(uint4 *) (s + r * kGenPitch + 16 * (tid & 7)) = v;
         }
     };
 
@@ -1876,29 +1918,42 @@ __global__ __launch_bounds__(kF32Threads) void gemm_f32(GemmParams p, float * pa
     __syncthreads();
     for (int step = 0; step < nsteps; ++step) {
         if (step + 1 < nsteps) load(step + 1);
-        const float * cur = st[step & 1];
+        const char * cur = st[step & 1];
 #pragma unroll
-        for (int q = 0; q < kF32BK / 16; ++q) {
-            f32x4_t wa[RG], xa[NT];
+        for (int q = 0; q < 2; ++q) {
+            uint4 wa[RG], xa[NT];
 #pragma unroll
             for (int rg = 0; rg < RG; ++rg)
-                wa[rg] = *(const f32x4_t *) (cur + (BM + 16 * (RG * wave + rg) + r16) * kF32Pitch + 16 * q + 4 * g);
+                wa[rg] = *(const uint4 *) (cur + (BM + 16 * (RG * wave + rg) + r16) * kGenPitch + 64 * q + 16 * g);
 #pragma unroll
             for (int t = 0; t < NT; ++t)
-                xa[t] = *(const f32x4_t *) (cur + (16 * t + r16) * kF32Pitch + 16 * q + 4 * g);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
+                xa[t] = *(const uint4 *) (cur + (16 * t + r16) * kGenPitch + 64 * q + 16 * g);
+            if constexpr (WBF) {
 #pragma unroll
                 for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
                     for (int t = 0; t < NT; ++t)
-                        acc[rg][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[t][e], wa[rg][e], acc[rg][t], 0, 0, 0);
+                        acc[rg][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            __builtin_bit_cast(bf16x8_t, xa[t]), __builtin_bit_cast(bf16x8_t, wa[rg]), acc[rg][t], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int rg = 0; rg < RG; ++rg)
+#pragma unroll
+                        for (int t = 0; t < NT; ++t)
+                            acc[rg][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                __builtin_bit_cast(f32x4_t, xa[t])[e], __builtin_bit_cast(f32x4_t, wa[rg])[e],
+                                acc[rg][t], 0, 0, 0);
+            }
         }
         if (step + 1 < nsteps) store(step + 1, st[(step + 1) & 1]);
         __syncthreads();
     }
-    char * y = (char *) p.y + (b2 * p.y_bs2 + b3 * p.y_bs3) * (p.y_type == WAMX_TYPE_F32 ? 4 : 2);
-    float * pp = part ? part + (int64_t) blockIdx.y * p.N * p.M : nullptr;
+    const int64_t yo = b2 * p.y_bs2 + b3 * p.y_bs3;
+    char * y = (char *) p.y + yo * (p.y_type == WAMX_TYPE_F32 ? 4 : 2);
+    const uint16_t * resb = p.res ? p.res + yo : nullptr;
+    float * pp = part ? part + ((int64_t) blockIdx.y * gridDim.z + blockIdx.z) * p.N * p.M : nullptr;
 #pragma unroll
     for (int rg = 0; rg < RG; ++rg) {
         const int64_t m = m0 + 16 * (RG * wave + rg) + r16;
@@ -1910,7 +1965,7 @@ __global__ __launch_bounds__(kF32Threads) void gemm_f32(GemmParams p, float * pa
                 const int64_t n = n0 + 16 * t + 4 * g + r;
                 if (n >= p.N) continue;
                 if (pp) pp[n * p.M + m] = acc[rg][t][r];
-                else store_out(p, y, p.res, n, m, acc[rg][t][r]);
+                else store_out(p, y, resb, n, m, acc[rg][t][r]);
             }
     }
 }
@@ -2280,72 +2335,88 @@ __global__ void round_rows_bf16_kernel(const float * __restrict__ x, int64_t ldx
     *(uint4 *) (y + r * K + 8 * c) = pack8(v);
 }
 
-// Tile and K split of an f32 product: the tokens in blocks of 16 NT with the
-// least padding, then the feature block (64 or 128) and the slice count with
-// the least modelled time, in us.  A workgroup's K step costs its MFMAs (32
+// Tile and K split of gemm_gen: the tokens in blocks of 16 NT with the least
+// padding, then the feature block (64 or 128) and the slice count with the
+// least modelled time, in us.  A workgroup's K step costs its MFMAs (f32: 32
 // cycles each on its SIMD) or its share of the weight stream, and 0.6 of load
 // latency that only a second workgroup of the CU hides; a split adds the
-// partials' traffic and the reduce.  Weights from HBM, sweep of both
+// partials' traffic and the reduce.  f32 weights from HBM, sweep of both
 // parameters: 3072 x 48 x 3072 26.8 us in 16 slices of 64 features against
 // 32.6 in 5, 14336 x 48 x 3072 67 in 3 or 4 slices against 92 unsplit, 3072 x
 // 121 x 3072 45 in 10 slices against 55 in 20; the model's choice is within a
 // tenth of each shape's best (times with a graph launch of one node).
-static void f32_plan(const GemmParams & p, bool may_split, size_t ws_bytes, int & nt, int & rg, int & splits, int & ks) {
+static void gen_plan(const GemmParams & p, bool wbf, int64_t batches, bool may_split, size_t ws_bytes, int & nt,
+                     int & rg, int & splits, int & ks) {
     if (p.N <= 64) nt = (int) ((p.N + 15) / 16);
     else nt = (p.N + 127) / 128 * 128 > (p.N + 63) / 64 * 64 ? 4 : 8;
-    const int64_t steps = (p.K + kF32BK - 1) / kF32BK;
+    const int bk = wbf ? 64 : 32;
+    const int64_t steps = (p.K + bk - 1) / bk;
     const int64_t nb = (p.N + 16 * nt - 1) / (16 * nt);
+    const double out = (double) p.N * (double) p.M * (double) batches;
     double best = 1e30;
     rg = nt == 8 ? 2 : 1;
     splits = 1;
-    ks = (int) steps * kF32BK;
-    for (int r = nt == 8 ? 2 : 1; r <= 2; ++r)
+    ks = (int) steps * bk;
+    for (int r = rg; r <= 2; ++r)
         for (int64_t sp = 1; sp <= (may_split ? 32 : 1); ++sp) {
             const int64_t per = (steps + sp - 1) / sp, s = (steps + per - 1) / per;
-            if (s != sp || (sp > 1 && (per < 4 || (size_t) sp * p.N * p.M * sizeof(float) > ws_bytes))) continue;
-            const double wgs = (double) nb * (double) ((p.M + 64 * r - 1) / (64 * r)) * (double) sp;
-            const double step = std::max(0.12 * nt, 0.36) * r;
+            if (s != sp || (sp > 1 && (per < 4 || (double) sp * out * 4 > (double) ws_bytes))) continue;
+            const double wgs = (double) nb * (double) ((p.M + 64 * r - 1) / (64 * r)) * (double) (sp * batches);
+            const double step = std::max((wbf ? 0.03 : 0.12) * nt, 0.36) * r;
             double t = (double) per * std::max(std::ceil(wgs / 256) * step, step + 0.6);
-            if (sp > 1) t += (double) sp * (double) p.N * (double) p.M * 8 / 4e6 + 3.0;
+            if (sp > 1) t += (double) sp * out * 8 / 4e6 + 3.0;
             if (t < best) {
                 best = t;
                 rg = r;
                 splits = (int) sp;
-                ks = (int) per * kF32BK;
+                ks = (int) per * bk;
             }
         }
 }
 
-static hipError_t run_f32(const GemmArgs & a, const GemmParams & p, hipStream_t s) {
-    const bool xbf = a.x_type == WAMX_TYPE_BF16;
-    if (!xbf && a.x_type != WAMX_TYPE_F32) return hipErrorInvalidValue;
-    const bool vec = !xbf && a.K % 4 == 0 && a.ldw % 4 == 0 && a.ldx % 4 == 0 && aligned16(a.w) && aligned16(a.x) &&
-                     a.w_bs2 % 4 == 0 && a.w_bs3 % 4 == 0 && a.x_bs2 % 4 == 0 && a.x_bs3 % 4 == 0;
-    const int64_t batches = a.B2 * a.B3;
-    int nt, rg, splits, ks;
-    f32_plan(p, batches == 1 && a.ws && aligned16(a.ws), a.ws_bytes, nt, rg, splits, ks);
-    const int nt_m = (int) ((p.M + 64 * rg - 1) / (64 * rg)), nt_n = (int) ((p.N + 16 * nt - 1) / (16 * nt));
-    const dim3 grid((unsigned) (nt_m * nt_n), (unsigned) splits, (unsigned) batches);
-    float * part = splits > 1 ? (float *) a.ws : nullptr;
-#define WAMX_F32(NT, RG)                                                                                               \
-    do {                                                                                                               \
-        if (vec) hipLaunchKernelGGL((gemm_f32<NT, RG, true, false>), grid, dim3(kF32Threads), 0, s, p, part, nt_m, nt_n, ks); \
-        else if (xbf) hipLaunchKernelGGL((gemm_f32<NT, RG, false, true>), grid, dim3(kF32Threads), 0, s, p, part, nt_m, nt_n, ks); \
-        else hipLaunchKernelGGL((gemm_f32<NT, RG, false, false>), grid, dim3(kF32Threads), 0, s, p, part, nt_m, nt_n, ks); \
-    } while (0)
-    switch (nt * 2 + rg - 1) {
-        case 2: WAMX_F32(1, 1); break;
-        case 3: WAMX_F32(1, 2); break;
-        case 4: WAMX_F32(2, 1); break;
-        case 5: WAMX_F32(2, 2); break;
-        case 6: WAMX_F32(3, 1); break;
-        case 7: WAMX_F32(3, 2); break;
-        case 8: WAMX_F32(4, 1); break;
-        case 9: WAMX_F32(4, 2); break;
-        default: WAMX_F32(8, 2); break;
+template <int NT, int RG>
+static void launch_gen(const GemmParams & p, bool wbf, bool xc, float * part, int splits, int64_t batches, int ks,
+                       hipStream_t s) {
+    const int nt_m = (int) ((p.M + 64 * RG - 1) / (64 * RG)), nt_n = (int) ((p.N + 16 * NT - 1) / (16 * NT));
+    const dim3 grid((unsigned) (nt_m * nt_n), (unsigned) splits, (unsigned) batches), block(kGenThreads);
+    if constexpr (NT <= 4) {
+        if (wbf) {
+            if (xc) hipLaunchKernelGGL((gemm_gen<NT, RG, true, true>), grid, block, 0, s, p, part, nt_m, nt_n, ks);
+            else hipLaunchKernelGGL((gemm_gen<NT, RG, true, false>), grid, block, 0, s, p, part, nt_m, nt_n, ks);
+            return;
+        }
     }
-#undef WAMX_F32
-    if (splits > 1) launch_reduce(p, part, splits, s);
+    if (xc) hipLaunchKernelGGL((gemm_gen<NT, RG, false, true>), grid, block, 0, s, p, part, nt_m, nt_n, ks);
+    else hipLaunchKernelGGL((gemm_gen<NT, RG, false, false>), grid, block, 0, s, p, part, nt_m, nt_n, ks);
+}
+
+// f32 weights, or bf16 weights with at most 64 tokens.
+static hipError_t run_gen(const GemmArgs & a, const GemmParams & p, hipStream_t s) {
+    const bool wbf = a.w_type == WAMX_TYPE_BF16, xbf = a.x_type == WAMX_TYPE_BF16;
+    if (!xbf && a.x_type != WAMX_TYPE_F32) return hipErrorInvalidValue;
+    const int64_t batches = a.B2 * a.B3;
+    // The partials' reduce walks the batches' outputs as one matrix.
+    const bool flat = batches == 1 || (a.epi == WAMX_EPI_NONE && a.ldy == a.M && a.y_bs2 == a.N * a.M &&
+                                       (a.B3 == 1 || a.y_bs3 == a.B2 * a.y_bs2));
+    int nt, rg, splits, ks;
+    gen_plan(p, wbf, batches, flat && a.ws && aligned16(a.ws), a.ws_bytes, nt, rg, splits, ks);
+    float * part = splits > 1 ? (float *) a.ws : nullptr;
+    switch (nt * 2 + rg - 1) {
+        case 2: launch_gen<1, 1>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
+        case 3: launch_gen<1, 2>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
+        case 4: launch_gen<2, 1>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
+        case 5: launch_gen<2, 2>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
+        case 6: launch_gen<3, 1>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
+        case 7: launch_gen<3, 2>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
+        case 8: launch_gen<4, 1>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
+        case 9: launch_gen<4, 2>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
+        default: launch_gen<8, 2>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
+    }
+    if (splits > 1) {
+        GemmParams q = p;
+        q.N = p.N * batches;
+        launch_reduce(q, part, splits, s);
+    }
     return hipGetLastError();
 }
 
@@ -2367,7 +2438,7 @@ hipError_t launch_gemm(const GemmArgs & a, hipStream_t s) {
     if (a.M <= 0 || a.N <= 0 || batches <= 0) return hipSuccess;
     if (a.K <= 0) return hipErrorInvalidValue;
 
-    if (a.w_type == WAMX_TYPE_F32) return run_f32(a, p, s);
+    if (a.w_type == WAMX_TYPE_F32) return run_gen(a, p, s);
     if (a.w_type != WAMX_TYPE_BF16 || (a.x_type != WAMX_TYPE_BF16 && a.x_type != WAMX_TYPE_F32))
         return hipErrorInvalidValue;
     const bool xf32 = a.x_type == WAMX_TYPE_F32;
@@ -2380,6 +2451,9 @@ hipError_t launch_gemm(const GemmArgs & a, hipStream_t s) {
         allow_skinny_lds();
         return run_skinny(p, xf32, a.w_tiled, a.ws, a.ws_bytes, s);
     }
+    // Few tokens in batches or with unaligned rows (the tiles below would pad
+    // them to 128 and leave most CUs idle).
+    if (a.N <= 64) return run_gen(a, p, s);
     if (vec && !xf32 && batches == 1) {
         hipError_t err = hipSuccess;
         if (dispatch_dma(p, a.ws, a.ws_bytes, s, err)) return err;
