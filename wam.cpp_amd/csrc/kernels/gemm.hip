@@ -9,12 +9,12 @@
 // Three kernels:
 //  * gemm_tile   — MFMA 32x32x16 bf16, LDS double-buffered 128x128x64 tiles,
 //                  128-bit global loads, for token counts above 64.
-//  * gemm_skinny — N <= 64 tokens (the 48-token action expert): HBM-bound
-//                  weight streaming with MFMA 16x16x32, K split across the
-//                  waves of a workgroup and reduced in LDS.
-//  * gemm_gen    — f32 weights (the f32 reference profile, generic MUL_MAT) on
-//                  f32 MFMA 16x16x4, and the few-token bf16 products in
-//                  batches or with unaligned rows.
+//  * gemm_skinny_tiled, gemm_skinny_wk — N <= 64 tokens (the 48-token action
+//                  expert) on tiled weights: HBM-bound weight streaming with
+//                  MFMA 16x16x32.
+//  * gemm_gen    — N <= 64 tokens on row-major weights, batches and any
+//                  alignment included, and f32 weights (the f32 reference
+//                  profile, generic MUL_MAT) on f32 MFMA 16x16x4.
 #include "../internal.h"
 #include "device.h"
 #include "rowops.h"
@@ -996,31 +996,24 @@ __global__ __launch_bounds__(64 * WM * WN * (SCHED == kSchedProducer ? 2 : 1), 1
 }
 
 // ---------------------------------------------------------------------------
-// gemm_skinny: N <= 64 tokens (the 48-token action expert), HBM-bound weight
-// streaming in two kernels.
+// gemm_skinny_tiled: N <= 64 tokens (the 48-token action expert) on tiled
+// weights (row-major ones take gemm_gen), HBM-bound weight streaming in two
+// kernels.
 //
-// gemm_skinny_part: grid = (feature blocks of 128) x (K splits).  The
-//   workgroup stages its K slice of the activations (all tokens, bf16) in LDS
-//   once, issuing every load of a batch before the first LDS store so the
-//   staging costs one memory latency, not one per chunk.  Each of its 8 waves
-//   then streams 16 weight rows of the slice from HBM with a 4-step-deep
-//   branch-free prefetch, and per 128-column step reads all activation
-//   fragments from LDS before feeding MFMA 16x16x32.  Activation bytes per
-//   workgroup are 48/128 of its weight bytes.  With one K split the epilogue
-//   is applied directly; otherwise fp32 partials go to a workspace.
+// The part kernel: grid = (feature blocks) x (K splits).  The workgroup stages
+//   its K slice of the activations (all tokens, bf16) in LDS once, issuing
+//   every load of a batch before the first LDS store so the staging costs one
+//   memory latency, not one per chunk.  Each wave then streams 16 weight rows
+//   of the slice with a branch-free prefetch, and per 128-column step reads
+//   all activation fragments from LDS before feeding MFMA 16x16x32.  With one
+//   K split the epilogue is applied directly; otherwise fp32 partials go to a
+//   workspace.
 // gemm_skinny_reduce: sums the K-split partials in split order
 //   (deterministic) and applies the epilogue, four outputs per thread with
 //   the split loads issued in batches of eight.  The kernel boundary orders
 //   the partial writes before the reads; no device-scope fences are needed.
-// Inside a 128-wide K step, MFMA chunk c of lane group g covers columns
-// 32c + 8g .. +8, so one load instruction reads 64 contiguous bytes of each
-// of its 16 weight rows (the activation fragments use the same order).
 // ---------------------------------------------------------------------------
-constexpr int kSkinnyWaves = 8;
-constexpr int kSkinnyRows = 32;                            // weight rows per wave (two MFMA groups)
-constexpr int kSkinnyFeat = kSkinnyRows * kSkinnyWaves;   // features per workgroup
-constexpr int kSkinnyDepth = 2;                            // weight prefetch depth (128-wide steps)
-constexpr int kSkinnyMaxKs = 1024;                         // longest K slice (LDS permitting)
+constexpr int kSkinnyDepth = 2;  // weight prefetch depth (128-wide steps)
 constexpr size_t kSkinnyLdsMax = 160 * 1024;
 
 // Stages x[0..N)[kb..kb+klen) as bf16 in LDS rows of ks + 8 elements (rows
@@ -1080,101 +1073,6 @@ __device__ __forceinline__ void skinny_store(const GemmParams & p, float * part,
     }
 }
 
-template <bool XF32, int NT, int DEPTH = kSkinnyDepth>
-__global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_skinny_part(GemmParams p, float * part, int ks) {
-    constexpr int RG = kSkinnyRows / 16;             // 16-row MFMA groups per wave
-    constexpr int LI = kSkinnyRows / 4;              // load instructions per step (4 rows x 256 B each)
-    extern __shared__ __align__(16) uint16_t xs[];  // [16*NT][ks + 8], then per-wave weight tiles
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = lane >> 4, r16 = lane & 15;
-    const int64_t M = p.M, K = p.K;
-    const int pitch = ks + 8;
-    const int64_t m0 = (int64_t) blockIdx.x * kSkinnyFeat + (int64_t) wave * kSkinnyRows;
-    const int64_t kb = (int64_t) blockIdx.y * ks;
-    const int64_t ke = min(K, kb + ks);
-    const int klen = (int) (ke - kb);
-    // Wave-private weight tile: kSkinnyRows rows x 128 columns, 16-byte chunk j
-    // of row r stored at chunk position j ^ (r & 15) (conflict-free row writes
-    // and column reads).
-    uint16_t * wt = xs + 16 * NT * pitch + wave * (kSkinnyRows * 128);
-
-    // Weight loads, row-coalesced: instruction c of a 128-column step reads
-    // rows 4c .. 4c+3 of the wave's rows, 256 contiguous bytes each (16 lanes
-    // per row).  Columns past the slice are clamped into it and masked to zero.
-    const int lrow = g, lchunk = r16;
-    const uint16_t * wbase[LI];
-#pragma unroll
-    for (int c = 0; c < LI; ++c) wbase[c] = p.w + min(m0 + 4 * c + lrow, M - 1) * p.ldw + kb;
-    const int nsteps = (klen + 127) / 128;
-    uint4 wbuf[DEPTH][LI];
-    // The loads only fill registers; the K-tail mask is applied where the
-    // values are consumed (any use of a loaded register right after the load
-    // would make the wave wait for it and serialise the prefetch).
-    auto wload = [&](int st, uint4 (&d)[LI]) {
-        const int k = st * 128 + 8 * lchunk;
-        const int kc = k < klen ? k : klen - 8;
-#pragma unroll
-        for (int c = 0; c < LI; ++c) d[c] = *(const uint4 *) (wbase[c] + kc);
-    };
-    skinny_stage_x<XF32>(p, xs, 16 * NT, ks, kb, klen, [&]() {
-#pragma unroll
-        for (int i = 0; i < DEPTH; ++i) wload(min(i, nsteps - 1), wbuf[i]);
-    });
-
-    f32x4_t acc[RG][NT];
-#pragma unroll
-    for (int rg = 0; rg < RG; ++rg)
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[rg][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    const uint16_t * xrow = xs + r16 * pitch + 8 * g;
-    for (int st0 = 0; st0 < nsteps; st0 += DEPTH) {
-#pragma unroll
-        for (int i = 0; i < DEPTH; ++i) {
-            const int st = st0 + i;
-            if (st < nsteps) {
-                // registers -> wave tile (row 4c + lrow, chunk lchunk); columns
-                // past the slice are zeroed here.
-                const uint32_t mask = st * 128 + 8 * lchunk < klen ? 0xffffffffu : 0u;
-#pragma unroll
-                for (int c = 0; c < LI; ++c) {
-                    const int r = 4 * c + lrow;
-                    const uint4 v = wbuf[i][c];
-                    *(uint4 *) (wt + r * 128 + ((lchunk ^ (r & 15)) << 3)) =
-                        make_uint4(v.x & mask, v.y & mask, v.z & mask, v.w & mask);
-                }
-                // MFMA chunk q: lane holds row r16 of group rg, columns 32q + 8g .. +8
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    bf16x8_t wa[RG], xa[NT];
-#pragma unroll
-                    for (int rg = 0; rg < RG; ++rg)
-                        wa[rg] = *(const bf16x8_t *) (wt + (16 * rg + r16) * 128 + (((4 * q + g) ^ r16) << 3));
-#pragma unroll
-                    for (int t = 0; t < NT; ++t)
-                        xa[t] = *(const bf16x8_t *) (xrow + 16 * t * pitch + st * 128 + 32 * q);
-#pragma unroll
-                    for (int rg = 0; rg < RG; ++rg)
-#pragma unroll
-                        for (int t = 0; t < NT; ++t)
-                            acc[rg][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[t], wa[rg], acc[rg][t], 0, 0, 0);
-                }
-            }
-            // Refilled on every pass (past the end with the last step again, an
-            // L2 hit), so every path issues the same loads and the wait before
-            // a slot's use counts only the younger slots' loads.
-            wload(min(st + DEPTH, nsteps - 1), wbuf[i]);
-        }
-    }
-    int64_t mrow[RG];
-    bool mok[RG];
-#pragma unroll
-    for (int rg = 0; rg < RG; ++rg) {
-        mrow[rg] = m0 + 16 * rg + r16;
-        mok[rg] = mrow[rg] < M;
-    }
-    skinny_store<RG, NT>(p, part, acc, mrow, mok, lane);
-}
-
 // ---------------------------------------------------------------------------
 // MFMA-tiled weights (the tiled buffer type): [M/16][K/32] tiles of 1 KB; in
 // tile (gr, q) lane l's 16 bytes are w[16 gr + (l & 15)][32 q + 8 (l >> 4) ..
@@ -1202,11 +1100,9 @@ hipError_t launch_tile_weights(const void * src, void * dst, int64_t M, int64_t 
     return hipGetLastError();
 }
 
-// gemm_skinny_part on tiled weights: each wave of the workgroup owns one
-// 16-row group (a workgroup of G waves covers 16 G features, G chosen with the
+// Each wave of the workgroup owns one 16-row group (a workgroup of G waves covers 16 G features, G chosen with the
 // K slice so the grid fills the CUs evenly), streams its tiles DEPTH steps
 // ahead and feeds them to the MFMAs as loaded, with no LDS on the weight path.
-// Within a K slice the accumulation order is that of gemm_skinny_part.
 // K % 32 == 0 and M % 16 == 0 (the tiled layout's conditions).
 constexpr int kTiledMaxWaves = 16;
 
@@ -1261,12 +1157,6 @@ __global__ __launch_bounds__(kTiledMaxWaves * 64) void gemm_skinny_tiled(GemmPar
     const int64_t mrow[1] = {16 * grp + r16};
     const bool mok[1] = {grp < ngrp};
     skinny_store<1, NT>(p, part, acc, mrow, mok, lane);
-}
-
-// LDS bytes of gemm_skinny_part: activation slice + the waves' weight tiles.
-static size_t skinny_lds_bytes(int nt, int ks) {
-    return (size_t) 16 * nt * (ks + 8) * sizeof(uint16_t) +
-           (size_t) kSkinnyWaves * kSkinnyRows * 128 * sizeof(uint16_t);
 }
 
 // V outputs per thread (V = 4 needs M % 4 == 0, so the four share a row).
@@ -1559,47 +1449,37 @@ __global__ __launch_bounds__(512) void skinny_reduce_row(GemmParams p, const flo
     }
 }
 
-// K split of the skinny path, from a small cost model (microseconds): the
-// slowest CU streams ceil(workgroups / 256) slices of kSkinnyFeat x ks
-// weights at its 1/256 share of 8 TB/s, plus a ramp per workgroup (one
-// workgroup per CU is resident: 8 waves of ~155 VGPRs); a split adds the fp32
-// partials (written and read once) and the reduce launch.  Measured on the
-// 48-token shapes this picks the fastest slice of the sweep for each.
-static void skinny_plan(int64_t M, int64_t N, int64_t K, int & splits, int & ks) {
-    const int64_t nfb = (M + kSkinnyFeat - 1) / kSkinnyFeat;
-    const int64_t nt = (N + 15) / 16;
+// Split-K partials that a few-token product with row-major weights may ask
+// for: the limit that callers' workspaces are checked against (products past
+// it have always been refused).  It is the fastest split of 256-feature
+// workgroups under a small cost model in microseconds: ceil(workgroups / 256)
+// slices of 256 x ks weights per CU at its 1/256 share of 8 TB/s, a ramp per
+// workgroup, the partials written and read once and the reduce launch.
+// gemm_gen's own plan (gen_plan) asks for no more than kGenPartBytes.
+size_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    const int64_t nfb = (M + 255) / 256, nt = (N + 15) / 16;
     double best = 1e30;
-    splits = (int) ((K + 127) / 128);
-    ks = 128;
-    for (int k = 128; k <= kSkinnyMaxKs; k += 128) {
+    int64_t splits = (K + 127) / 128;
+    for (int64_t k = 128; k <= 1024; k += 128) {
         const int64_t s = (K + k - 1) / k;
-        if (s > 1 && (int64_t) k * (s - 1) >= K) continue;
-        const size_t lds = skinny_lds_bytes((int) nt, k);
-        if (lds > kSkinnyLdsMax) break;
-        const int64_t wgs = nfb * s;
-        const int64_t per_cu = (wgs + 255) / 256;
-        double t = per_cu * ((double) kSkinnyFeat * std::min<int64_t>(k, K) * 2 / 31.25e3 + 1.5);
-        if (s > 1) t += (double) s * N * M * 4 * 2 / 8e6 + 3.0;
+        if (s > 1 && k * (s - 1) >= K) continue;
+        if ((16 * nt * (k + 8) + 256 * 128) * 2 > 160 * 1024) break;
+        double t = (double) ((nfb * s + 255) / 256) * (256.0 * (double) std::min(k, K) * 2 / 31.25e3 + 1.5);
+        if (s > 1) t += (double) s * (double) N * (double) M * 4 * 2 / 8e6 + 3.0;
         if (t < best) {
             best = t;
-            splits = (int) s;
-            ks = k;
+            splits = s;
         }
         if (k >= K) break;
     }
-}
-
-size_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    int splits, ks;
-    skinny_plan(M, N, K, splits, ks);
     return splits > 1 ? (size_t) splits * N * M * sizeof(float) : 0;
 }
 
 static int64_t tiles_of(const GemmParams & p, int bm, int bn);
 static int dma_splitk_plan(const GemmParams & p, size_t ws_bytes);
 
-// The K split launch_gemm takes for a plain product with row-major weights:
-// the skinny plan up to 64 tokens, else the K-sliced 128 x 128 GEMM that
+// The K split of a plain product with row-major weights: the few-token limit
+// up to 64 tokens, else the K-sliced 128 x 128 GEMM that
 // dispatch_dma runs for bf16 activations on grids too small for the 256 /
 // 192 tiles (whose slice count depends on the workspace size).
 size_t linear_split_bytes(int64_t M, int64_t N, int64_t K, int32_t x_type, size_t ws_bytes) {
@@ -1615,8 +1495,6 @@ size_t linear_split_bytes(int64_t M, int64_t N, int64_t K, int32_t x_type, size_
     return splits > 1 ? (size_t) splits * N * M * sizeof(float) : 0;
 }
 
-// gemm_skinny_part over `splits` K slices of ks columns; part == nullptr
-// (single slice only) applies the epilogue in the part kernel.
 // Workgroup shape of the tiled kernel: G waves (16 G features) by a K slice
 // of ks columns.  Measured on the action expert's projections (48 and 1
 // tokens, part + reduce, weights streamed from HBM) over G = 4..12 and ks =
@@ -1643,7 +1521,7 @@ static void skinny_tiled_plan(int64_t M, int64_t N, int64_t K, int & splits, int
     const int64_t kwhole = (K + 127) / 128 * 128;  // one slice over all of K
     splits = (int) ((K + 383) / 384);
     ks = 384;
-    waves = kSkinnyWaves;
+    waves = 8;
     // Slices of 384..1536 columns, or all of a shorter K in one.  One always
     // fits the LDS (a 16 x 64-token activation slice of 384 columns is 49 KB),
     // and with G = 4 every grid fits some number of rounds, so the search
@@ -1669,42 +1547,21 @@ static void skinny_tiled_plan(int64_t M, int64_t N, int64_t K, int & splits, int
     }
 }
 
-static void skinny_plan_for(const GemmParams & p, bool tiled, int & splits, int & ks, int & waves) {
-    waves = kSkinnyWaves;
-    if (tiled) skinny_tiled_plan(p.M, p.N, p.K, splits, ks, waves);
-    else skinny_plan(p.M, p.N, p.K, splits, ks);
-}
-
-// gemm_skinny_part (or gemm_skinny_tiled) over `splits` K slices of ks
-// columns; part == nullptr (single slice only) applies the epilogue in the
-// part kernel.
-static void launch_skinny_part(const GemmParams & p, bool xf32, bool tiled, float * part, int splits, int ks,
-                               int waves, hipStream_t s) {
+// gemm_skinny_tiled over `splits` K slices of ks columns; part == nullptr
+// (single slice only) applies the epilogue in the part kernel.
+static void launch_skinny_part(const GemmParams & p, bool xf32, float * part, int splits, int ks, int waves,
+                               hipStream_t s) {
     const int nt = (int) ((p.N + 15) / 16);
-    const dim3 block(kSkinnyWaves * 64);
-    if (tiled) {
-        const size_t lds = (size_t) 16 * nt * (ks + 8) * sizeof(uint16_t);
-        const dim3 grid((unsigned) ((p.M / 16 + waves - 1) / waves), (unsigned) splits), tblock((unsigned) (64 * waves));
+    const size_t lds = (size_t) 16 * nt * (ks + 8) * sizeof(uint16_t);
+    const dim3 grid((unsigned) ((p.M / 16 + waves - 1) / waves), (unsigned) splits), tblock((unsigned) (64 * waves));
 #define WAMX_TILED(XF, NT) hipLaunchKernelGGL((gemm_skinny_tiled<XF, NT>), grid, tblock, lds, s, p, part, ks)
-        switch (nt) {
-            case 1: if (xf32) WAMX_TILED(true, 1); else WAMX_TILED(false, 1); break;
-            case 2: if (xf32) WAMX_TILED(true, 2); else WAMX_TILED(false, 2); break;
-            case 3: if (xf32) WAMX_TILED(true, 3); else WAMX_TILED(false, 3); break;
-            default: if (xf32) WAMX_TILED(true, 4); else WAMX_TILED(false, 4); break;
-        }
-#undef WAMX_TILED
-        return;
-    }
-    const size_t lds = skinny_lds_bytes(nt, ks);
-    const dim3 grid((unsigned) ((p.M + kSkinnyFeat - 1) / kSkinnyFeat), (unsigned) splits);
-#define WAMX_SKINNY(XF, NT) hipLaunchKernelGGL((gemm_skinny_part<XF, NT>), grid, block, lds, s, p, part, ks)
     switch (nt) {
-        case 1: if (xf32) WAMX_SKINNY(true, 1); else WAMX_SKINNY(false, 1); break;
-        case 2: if (xf32) WAMX_SKINNY(true, 2); else WAMX_SKINNY(false, 2); break;
-        case 3: if (xf32) WAMX_SKINNY(true, 3); else WAMX_SKINNY(false, 3); break;
-        default: if (xf32) WAMX_SKINNY(true, 4); else WAMX_SKINNY(false, 4); break;
+        case 1: if (xf32) WAMX_TILED(true, 1); else WAMX_TILED(false, 1); break;
+        case 2: if (xf32) WAMX_TILED(true, 2); else WAMX_TILED(false, 2); break;
+        case 3: if (xf32) WAMX_TILED(true, 3); else WAMX_TILED(false, 3); break;
+        default: if (xf32) WAMX_TILED(true, 4); else WAMX_TILED(false, 4); break;
     }
-#undef WAMX_SKINNY
+#undef WAMX_TILED
 }
 
 // WAMX_DISABLE_SKINNY_WK=1 keeps the split-K path for these products (read at
@@ -1717,9 +1574,9 @@ static bool skinny_wk_enabled() {
 // Whether gemm_skinny_wk takes the product: tiled weights, bf16 activations
 // and output with the vector epilogue, 64-feature groups filling most of the
 // CUs, and whole k-tile steps per wave.
-static bool skinny_wk_ok(const GemmParams & p, bool xf32, bool tiled) {
+static bool skinny_wk_ok(const GemmParams & p, bool xf32) {
     const int64_t kt = p.K / 32;
-    return tiled && !xf32 && p.vec_out && epi_kind(p) != kEpiF32 && p.N <= 64 && p.M % (16 * kWkGroups) == 0 &&
+    return !xf32 && p.vec_out && epi_kind(p) != kEpiF32 && p.N <= 64 && p.M % (16 * kWkGroups) == 0 &&
            p.M / (16 * kWkGroups) >= 192 && p.K % 32 == 0 && kt % kWkWaves == 0 && (kt / kWkWaves) % kWkDepth == 0;
 }
 
@@ -1745,8 +1602,9 @@ static void launch_reduce(const GemmParams & p, const float * part, int splits, 
                            splits);
 }
 
-static hipError_t run_skinny(const GemmParams & p, bool xf32, bool tiled, void * ws, size_t ws_bytes, hipStream_t s) {
-    if (skinny_wk_ok(p, xf32, tiled) && skinny_wk_enabled()) {
+// Tiled weights.
+static hipError_t run_skinny(const GemmParams & p, bool xf32, void * ws, size_t ws_bytes, hipStream_t s) {
+    if (skinny_wk_ok(p, xf32) && skinny_wk_enabled()) {
         switch ((p.N + 15) / 16) {
             case 1: launch_skinny_wk<1>(p, s); break;
             case 2: launch_skinny_wk<2>(p, s); break;
@@ -1756,25 +1614,24 @@ static hipError_t run_skinny(const GemmParams & p, bool xf32, bool tiled, void *
         return hipGetLastError();
     }
     int splits, ks, waves;
-    skinny_plan_for(p, tiled, splits, ks, waves);
+    skinny_tiled_plan(p.M, p.N, p.K, splits, ks, waves);
     if (splits > 1 && (!ws || (size_t) splits * p.N * p.M * sizeof(float) > ws_bytes || ((uintptr_t) ws & 15)))
         return hipErrorInvalidValue;
     float * part = splits > 1 ? (float *) ws : nullptr;
-    launch_skinny_part(p, xf32, tiled, part, splits, ks, waves, s);
+    launch_skinny_part(p, xf32, part, splits, ks, waves, s);
     if (splits > 1) launch_reduce(p, part, splits, s);
     return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
-// gemm_gen: the products the LDS-DMA and skinny kernels do not take: f32
-// weights at any size (the f32 reference profile, MUL_MAT of two f32 tensors,
-// f32 convolutions; products and sums in f32 on MFMA 16x16x4), and bf16
-// weights at up to 64 tokens in batches or with rows of any alignment
-// (attention of separate ggml nodes; MFMA 16x16x32).
+// gemm_gen: row-major bf16 weights at up to 64 tokens, in batches or with rows
+// of any alignment too (attention of separate ggml nodes; MFMA 16x16x32), and
+// f32 weights at any size (the f32 reference profile, MUL_MAT of two f32
+// tensors, f32 convolutions; products and sums in f32 on MFMA 16x16x4).
 //
 // A workgroup of 4 waves multiplies 16 NT tokens by 64 RG features.  A K step
 // is 128 bytes of each weight row (32 f32 or 64 bf16), through two LDS stages
-// with the next step's loads held in registers meanwhile.  Lane group g's
+// with the loads of the next D steps held in registers meanwhile.  Lane group g's
 // 16-byte fragments cover bytes 64 q + 16 g .. + 16 of both operands; in f32
 // one feeds 4 MFMAs, one column of each group per MFMA (both operands take the
 // same K order, so any order is a valid one).  Rows are padded by 16 bytes: 16
@@ -1808,14 +1665,21 @@ __device__ __forceinline__ uint4 load_loose16(const char * p) {
 
 // WBF: bf16 weights, else f32.  XC: activations of the other type, rounded to
 // bf16 or widened on their way into LDS.
-template <int NT, int RG, bool WBF, bool XC>
+template <int NT, int RG>
+constexpr int gen_depth() {
+    return NT > 4 ? 1 : RG == 2 ? 3 : 4;
+}
+template <int NT, int RG, bool WBF, bool XC, int D = gen_depth<NT, RG>()>
 __global__ __launch_bounds__(kGenThreads, 2) void gemm_gen(GemmParams p, float * part, int nt_m, int nt_n, int ks) {
     constexpr int BM = 16 * NT, BN = 64 * RG, ROWS = BM + BN;
     constexpr int EPC = WBF ? 8 : 4, BK = 8 * EPC;        // elements per 16-byte chunk, per step
     constexpr int WS = WBF ? 2 : 4, XS = XC ? 6 - WS : WS;  // element sizes
     constexpr int NL = (ROWS + 31) / 32;                   // 32 rows of 8 chunks per load instruction
     constexpr int NX = XC && WBF ? (BM + 31) / 32 : 1;     // second halves of f32 activations
-    __shared__ __align__(16) char st[2][ROWS * kGenPitch];
+    // Rows of a last part-full load instruction are copied too (the last weight
+    // row again): a load that some lanes did not use would have to be waited
+    // for before its registers serve another purpose.
+    __shared__ __align__(16) char st[2][NL * 32 * kGenPitch];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, r16 = lane & 15;
     const int64_t b2 = blockIdx.z % p.B2, b3 = blockIdx.z / p.B2;
@@ -1842,9 +1706,8 @@ __global__ __launch_bounds__(kGenThreads, 2) void gemm_gen(GemmParams p, float *
     // with it, and shifted into place on its way into LDS (columns left of the
     // slice are the row's own: K >= EPC).
     const int cb = EPC * (tid & 7);  // the chunk's first column in a step
-    uint4 raw[NL], raw2[NX];
-    auto load = [&](int step) {
-        if (p.K < EPC) return;
+    uint4 raws[D][NL], raws2[D][NX];
+    auto load = [&](int step, uint4 (&raw)[NL], uint4 (&raw2)[NX]) {
         const int64_t k = min(step * BK + cb, klen - EPC) - cb;
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
@@ -1861,25 +1724,8 @@ __global__ __launch_bounds__(kGenThreads, 2) void gemm_gen(GemmParams p, float *
             }
         }
     };
-    auto store = [&](int step, char * s) {
-        if (p.K < EPC) {  // a few columns in all: element by element
-#pragma unroll 1
-            for (int i = tid; i < ROWS * BK; i += kGenThreads) {
-                const int r = i / BK, c = i % BK;
-                uint32_t v = 0;
-                if (c < klen && r < BM) {
-                    const char * q = xt + ((int64_t) min(r, nlast) * p.ldx + c) * XS;
-                    if (XS == 4) v = WBF ? f32_to_bf16(*(const float *) q) : *(const uint32_t *) q;
-                    else v = (uint32_t) *(const uint16_t *) q << (WBF ? 0 : 16);
-                } else if (c < klen) {
-                    const char * q = wt + ((int64_t) min(r - BM, mlast) * p.ldw + c) * WS;
-                    v = WBF ? *(const uint16_t *) q : *(const uint32_t *) q;
-                }
-                if (WBF) *(uint16_t *) (s + r * kGenPitch + 2 * c) = (uint16_t) v;
-                else *(uint32_t *) (s + r * kGenPitch + 4 * c) = v;
-            }
-            return;
-        }
+    // The step's chunks into LDS; tail_c: the step that the slice ends in.
+    auto store = [&](auto tail_c, int step, char * s, const uint4 (&raw)[NL], const uint4 (&raw2)[NX]) {
         const int d = max(step * BK + cb - (klen - EPC), 0);  // elements to shift out
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
@@ -1896,7 +1742,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void gemm_gen(GemmParams p, float *
                     v = make_uint4(v.x << 16, v.x & 0xFFFF0000u, v.y << 16, v.y & 0xFFFF0000u);
                 }
             }
-            if (step * BK + BK > klen) {
+            if constexpr (decltype(tail_c)::value) {
                 const int dw = d * WS / 4;
                 if (dw & 1) v = make_uint4(v.y, v.z, v.w, 0);
                 if (dw & 2) v = make_uint4(v.z, v.w, 0, 0);
@@ -1904,7 +1750,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void gemm_gen(GemmParams p, float *
                     v = make_uint4(v.x >> 16 | v.y << 16, v.y >> 16 | v.z << 16, v.z >> 16 | v.w << 16, v.w >> 16);
                 if (d >= EPC) v = make_uint4(0, 0, 0, 0);
             }
-            if ((i + 1) * 32 <= ROWS || r < ROWS) *(uint4 *) (s + r * kGenPitch + 16 * (tid & 7)) = v;
+            *(uint4 *) (s + r * kGenPitch + 16 * (tid & 7)) = v;
         }
     };
 
@@ -1913,12 +1759,7 @@ __global__ __launch_bounds__(kGenThreads, 2) void gemm_gen(GemmParams p, float *
     for (int rg = 0; rg < RG; ++rg)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[rg][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    load(0);
-    store(0, st[0]);
-    __syncthreads();
-    for (int step = 0; step < nsteps; ++step) {
-        if (step + 1 < nsteps) load(step + 1);
-        const char * cur = st[step & 1];
+    auto mma = [&](const char * cur) {
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             uint4 wa[RG], xa[NT];
@@ -1947,8 +1788,55 @@ __global__ __launch_bounds__(kGenThreads, 2) void gemm_gen(GemmParams p, float *
                                 acc[rg][t], 0, 0, 0);
             }
         }
-        if (step + 1 < nsteps) store(step + 1, st[(step + 1) & 1]);
+    };
+    if (p.K < EPC) {  // a few columns in all: element by element
+#pragma unroll 1
+        for (int i = tid; i < ROWS * BK; i += kGenThreads) {
+            const int r = i / BK, c = i % BK;
+            uint32_t v = 0;
+            if (c < klen && r < BM) {
+                const char * q = xt + ((int64_t) min(r, nlast) * p.ldx + c) * XS;
+                if (XS == 4) v = WBF ? f32_to_bf16(*(const float *) q) : *(const uint32_t *) q;
+                else v = (uint32_t) *(const uint16_t *) q << (WBF ? 0 : 16);
+            } else if (c < klen) {
+                const char * q = wt + ((int64_t) min(r - BM, mlast) * p.ldw + c) * WS;
+                v = WBF ? *(const uint16_t *) q : *(const uint32_t *) q;
+            }
+            if (WBF) *(uint16_t *) (st[0] + r * kGenPitch + 2 * c) = (uint16_t) v;
+            else *(uint32_t *) (st[0] + r * kGenPitch + 4 * c) = v;
+        }
         __syncthreads();
+        mma(st[0]);
+    } else {
+        // One barrier per step: a stage is written again two steps later, when
+        // every wave is past the barrier that follows its reads.  Past the last
+        // step that one is loaded again, unused, so that every wait counts the
+        // same number of younger loads.
+#pragma unroll
+        for (int i = 0; i < D; ++i) load(min(i, nsteps - 1), raws[i], raws2[i]);
+        const int nfull = klen / BK;
+        auto run = [&](int step, uint4 (&raw)[NL], uint4 (&raw2)[NX]) {
+            store(std::false_type{}, step, st[step & 1], raw, raw2);
+            __syncthreads();
+            load(min(step + D, nsteps - 1), raw, raw2);
+            mma(st[step & 1]);
+        };
+        // Whole rounds of D steps, then the rest: in one loop the waits would
+        // have to cover leaving it in mid-round.
+        int step0 = 0;
+        for (; step0 + D <= nfull; step0 += D)
+#pragma unroll
+            for (int i = 0; i < D; ++i) run(step0 + i, raws[i], raws2[i]);
+#pragma unroll
+        for (int i = 0; i < D - 1; ++i)
+            if (step0 + i < nfull) run(step0 + i, raws[i], raws2[i]);
+        if (nfull < nsteps) {
+#pragma unroll
+            for (int i = 0; i < D; ++i)
+                if (nfull % D == i) store(std::true_type{}, nfull, st[nfull & 1], raws[i], raws2[i]);
+            __syncthreads();
+            mma(st[nfull & 1]);
+        }
     }
     const int64_t yo = b2 * p.y_bs2 + b3 * p.y_bs3;
     char * y = (char *) p.y + yo * (p.y_type == WAMX_TYPE_F32 ? 4 : 2);
@@ -2174,14 +2062,112 @@ static bool vec_operands(const GemmArgs & a) {
            a.w_bs3 % 8 == 0 && a.x_bs2 % 8 == 0 && a.x_bs3 % 8 == 0;
 }
 
+// Tile and K split of gemm_gen: the tokens in blocks of 16 NT with the least
+// padding, then the feature block (64 or 128) and the slice count with the
+// least modelled time, in us.  A workgroup's K step costs the bytes it copies
+// (29 ns per KB, weights and activations) or, in f32, its MFMAs (32 cycles
+// each on its SIMD); workgroups run in rounds of one per CU, since with D
+// steps of loads in flight a second one of a CU only divides its share; a
+// split adds the partials' traffic and the reduce launch.
+//
+// Sweep of both parameters, bf16 weights from HBM, both launches (us): 3072 x
+// 48 x 3072 13.1 in 4 slices of 64 features (192 workgroups) against 15.9 in 2
+// and 16 in 6; 14336 x 48 x 3072 23.1 unsplit (224) against 27.0 in 2 slices
+// of 128; 9216 x 48 x 3072 20.6 in 3 slices of 128 (216) against 26.0 in 4 of
+// 64; f32 activations, 10240 x 64 x 4096 33.1 in 3 slices of 128 (240) against
+// 41.0 in 3 of 64.  256-feature workgroups of 8 waves with the weights staged
+// per wave, two steps ahead, which this replaced for row-major weights, took
+// 20.2, 31.0, 24.6 and 45.5.
+constexpr size_t kGenPartBytes = 32ull << 20;
+struct GenPlan {
+    int nt, rg, splits, ks;
+};
+static GenPlan gen_plan(const GemmParams & p, bool wbf, bool xbf, int64_t batches, size_t ws_bytes) {
+    GenPlan b{};
+    if (p.N <= 64) b.nt = (int) ((p.N + 15) / 16);
+    else b.nt = (p.N + 127) / 128 * 128 > (p.N + 63) / 64 * 64 ? 4 : 8;
+    const int bk = wbf ? 64 : 32;
+    const int64_t steps = (p.K + bk - 1) / bk, nb = (p.N + 16 * b.nt - 1) / (16 * b.nt);
+    const double out = (double) p.N * (double) p.M * (double) batches;
+    const double limit = (double) std::min(ws_bytes, kGenPartBytes);
+    const double xkb = wbf == xbf ? 2 : wbf ? 4 : 1;  // KB of 16 tokens' step
+    double best = 1e30;
+    b.rg = b.nt == 8 ? 2 : 1;
+    b.splits = 1;
+    b.ks = (int) steps * bk;
+    for (int r = b.rg; r <= 2; ++r)
+        for (int64_t sp = 1; sp <= 32; ++sp) {
+            const int64_t per = (steps + sp - 1) / sp, s = (steps + per - 1) / per;
+            if (s != sp || (sp > 1 && (per < 4 || (double) sp * out * 4 > limit))) continue;
+            const double wgs = (double) nb * (double) ((p.M + 64 * r - 1) / (64 * r)) * (double) (sp * batches);
+            double step = std::max(0.029 * (8 * r + xkb * b.nt), wbf ? 0.0 : 0.12 * b.nt * r);
+            if (b.nt == 8) step += 0.6;  // one step in flight: its latency shows
+            double t = std::ceil(wgs / 256) * (double) per * step;
+            if (sp > 1) t += (double) sp * out * 8 / 4e6 + 4.0;
+            if (t < best) {
+                best = t;
+                b.rg = r;
+                b.splits = (int) sp;
+                b.ks = (int) per * bk;
+            }
+        }
+    return b;
+}
+
+template <int NT, int RG>
+static void launch_gen(const GemmParams & p, bool wbf, bool xc, float * part, const GenPlan & b, int64_t batches,
+                       hipStream_t s) {
+    const int nt_m = (int) ((p.M + 64 * RG - 1) / (64 * RG)), nt_n = (int) ((p.N + 16 * NT - 1) / (16 * NT));
+    const dim3 grid((unsigned) (nt_m * nt_n), (unsigned) b.splits, (unsigned) batches), block(kGenThreads);
+    if constexpr (NT <= 4) {
+        if (wbf) {
+            if (xc) hipLaunchKernelGGL((gemm_gen<NT, RG, true, true>), grid, block, 0, s, p, part, nt_m, nt_n, b.ks);
+            else hipLaunchKernelGGL((gemm_gen<NT, RG, true, false>), grid, block, 0, s, p, part, nt_m, nt_n, b.ks);
+            return;
+        }
+    }
+    if (xc) hipLaunchKernelGGL((gemm_gen<NT, RG, false, true>), grid, block, 0, s, p, part, nt_m, nt_n, b.ks);
+    else hipLaunchKernelGGL((gemm_gen<NT, RG, false, false>), grid, block, 0, s, p, part, nt_m, nt_n, b.ks);
+}
+// part: f32 partials, or null (one slice) for the epilogue in the kernel.
+static void launch_gen_part(const GemmParams & p, bool wbf, bool xbf, float * part, const GenPlan & b, int64_t batches,
+                            hipStream_t s) {
+    switch (b.nt * 2 + b.rg - 1) {
+        case 2: launch_gen<1, 1>(p, wbf, wbf != xbf, part, b, batches, s); break;
+        case 3: launch_gen<1, 2>(p, wbf, wbf != xbf, part, b, batches, s); break;
+        case 4: launch_gen<2, 1>(p, wbf, wbf != xbf, part, b, batches, s); break;
+        case 5: launch_gen<2, 2>(p, wbf, wbf != xbf, part, b, batches, s); break;
+        case 6: launch_gen<3, 1>(p, wbf, wbf != xbf, part, b, batches, s); break;
+        case 7: launch_gen<3, 2>(p, wbf, wbf != xbf, part, b, batches, s); break;
+        case 8: launch_gen<4, 1>(p, wbf, wbf != xbf, part, b, batches, s); break;
+        case 9: launch_gen<4, 2>(p, wbf, wbf != xbf, part, b, batches, s); break;
+        default: launch_gen<8, 2>(p, wbf, wbf != xbf, part, b, batches, s); break;
+    }
+}
+
+// f32 weights, or row-major bf16 weights with at most 64 tokens.
+static hipError_t run_gen(const GemmArgs & a, const GemmParams & p, hipStream_t s) {
+    const bool wbf = a.w_type == WAMX_TYPE_BF16, xbf = a.x_type == WAMX_TYPE_BF16;
+    if (!xbf && a.x_type != WAMX_TYPE_F32) return hipErrorInvalidValue;
+    const int64_t batches = a.B2 * a.B3;
+    // The partials' reduce walks the batches' outputs as one matrix.
+    const bool flat = batches == 1 || (a.epi == WAMX_EPI_NONE && a.ldy == a.M && a.y_bs2 == a.N * a.M &&
+                                       (a.B3 == 1 || a.y_bs3 == a.B2 * a.y_bs2));
+    const GenPlan b = gen_plan(p, wbf, xbf, batches, flat && a.ws && aligned16(a.ws) ? a.ws_bytes : 0);
+    float * part = b.splits > 1 ? (float *) a.ws : nullptr;
+    launch_gen_part(p, wbf, xbf, part, b, batches, s);
+    if (b.splits > 1) {
+        GemmParams q = p;
+        q.N = p.N * batches;
+        launch_reduce(q, part, b.splits, s);
+    }
+    return hipGetLastError();
+}
+
 static void allow_skinny_lds() {
-    // The activation slice and the weight tiles may use all 160 KB of LDS.
+    // The activation slice may use all 160 KB of LDS.
     constexpr size_t kMaxLds = kSkinnyLdsMax;
-    static bool once = (allow_lds(gemm_skinny_part<true, 1>, kMaxLds), allow_lds(gemm_skinny_part<false, 1>, kMaxLds),
-                        allow_lds(gemm_skinny_part<true, 2>, kMaxLds), allow_lds(gemm_skinny_part<false, 2>, kMaxLds),
-                        allow_lds(gemm_skinny_part<true, 3>, kMaxLds), allow_lds(gemm_skinny_part<false, 3>, kMaxLds),
-                        allow_lds(gemm_skinny_part<true, 4>, kMaxLds), allow_lds(gemm_skinny_part<false, 4>, kMaxLds),
-                        allow_lds(gemm_skinny_tiled<true, 1>, kMaxLds), allow_lds(gemm_skinny_tiled<false, 1>, kMaxLds),
+    static bool once = (allow_lds(gemm_skinny_tiled<true, 1>, kMaxLds), allow_lds(gemm_skinny_tiled<false, 1>, kMaxLds),
                         allow_lds(gemm_skinny_tiled<true, 2>, kMaxLds), allow_lds(gemm_skinny_tiled<false, 2>, kMaxLds),
                         allow_lds(gemm_skinny_tiled<true, 3>, kMaxLds), allow_lds(gemm_skinny_tiled<false, 3>, kMaxLds),
                         allow_lds(gemm_skinny_tiled<true, 4>, kMaxLds), allow_lds(gemm_skinny_tiled<false, 4>, kMaxLds),
@@ -2208,14 +2194,19 @@ hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStre
     // K-sliced 128 x 128 GEMM (its partial planes are the reduce's layout).
     const bool dma = a.N > 64;
     int splits = 1, ks = 0, waves = 0;
+    GenPlan gp{};
     if (dma) {
         if (a.w_tiled || a.x_type != WAMX_TYPE_BF16 || p.K % 64 != 0 || tiles_of(p, 256, 256) >= 256 ||
             tiles_of(p, 192, 192) >= 192)
             return hipErrorNotSupported;
         splits = dma_splitk_plan(p, a.ws_bytes);
         if (splits <= 1) return hipErrorNotSupported;
+    } else if (a.w_tiled) {
+        skinny_tiled_plan(p.M, p.N, p.K, splits, ks, waves);
     } else {
-        skinny_plan_for(p, a.w_tiled, splits, ks, waves);
+        if (skinny_workspace_bytes(p.M, p.N, p.K) > a.ws_bytes) return hipErrorNotSupported;
+        gp = gen_plan(p, true, a.x_type == WAMX_TYPE_BF16, 1, a.ws_bytes);
+        splits = gp.splits;
     }
     if ((size_t) splits * p.N * p.M * sizeof(float) > a.ws_bytes) return hipErrorNotSupported;
 
@@ -2294,9 +2285,11 @@ hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStre
     const float * part = (const float *) a.ws;
     if (dma) {
         launch_dma_splitk_parts(p, splits, a.ws, s);
-    } else {
+    } else if (a.w_tiled) {
         allow_skinny_lds();
-        launch_skinny_part(p, a.x_type == WAMX_TYPE_F32, a.w_tiled, (float *) a.ws, splits, ks, waves, s);
+        launch_skinny_part(p, a.x_type == WAMX_TYPE_F32, (float *) a.ws, splits, ks, waves, s);
+    } else {
+        launch_gen_part(p, true, a.x_type == WAMX_TYPE_BF16, (float *) a.ws, gp, 1, s);
     }
     const dim3 grid((unsigned) p.N, (unsigned) nseg), block((unsigned) nchunk);
 #define WAMX_ROW(EK, PK) hipLaunchKernelGGL((skinny_reduce_row<EK, PK>), grid, block, 0, s, p, part, splits, d)
@@ -2335,91 +2328,6 @@ __global__ void round_rows_bf16_kernel(const float * __restrict__ x, int64_t ldx
     *(uint4 *) (y + r * K + 8 * c) = pack8(v);
 }
 
-// Tile and K split of gemm_gen: the tokens in blocks of 16 NT with the least
-// padding, then the feature block (64 or 128) and the slice count with the
-// least modelled time, in us.  A workgroup's K step costs its MFMAs (f32: 32
-// cycles each on its SIMD) or its share of the weight stream, and 0.6 of load
-// latency that only a second workgroup of the CU hides; a split adds the
-// partials' traffic and the reduce.  f32 weights from HBM, sweep of both
-// parameters: 3072 x 48 x 3072 26.8 us in 16 slices of 64 features against
-// 32.6 in 5, 14336 x 48 x 3072 67 in 3 or 4 slices against 92 unsplit, 3072 x
-// 121 x 3072 45 in 10 slices against 55 in 20; the model's choice is within a
-// tenth of each shape's best (times with a graph launch of one node).
-static void gen_plan(const GemmParams & p, bool wbf, int64_t batches, bool may_split, size_t ws_bytes, int & nt,
-                     int & rg, int & splits, int & ks) {
-    if (p.N <= 64) nt = (int) ((p.N + 15) / 16);
-    else nt = (p.N + 127) / 128 * 128 > (p.N + 63) / 64 * 64 ? 4 : 8;
-    const int bk = wbf ? 64 : 32;
-    const int64_t steps = (p.K + bk - 1) / bk;
-    const int64_t nb = (p.N + 16 * nt - 1) / (16 * nt);
-    const double out = (double) p.N * (double) p.M * (double) batches;
-    double best = 1e30;
-    rg = nt == 8 ? 2 : 1;
-    splits = 1;
-    ks = (int) steps * bk;
-    for (int r = rg; r <= 2; ++r)
-        for (int64_t sp = 1; sp <= (may_split ? 32 : 1); ++sp) {
-            const int64_t per = (steps + sp - 1) / sp, s = (steps + per - 1) / per;
-            if (s != sp || (sp > 1 && (per < 4 || (double) sp * out * 4 > (double) ws_bytes))) continue;
-            const double wgs = (double) nb * (double) ((p.M + 64 * r - 1) / (64 * r)) * (double) (sp * batches);
-            const double step = std::max((wbf ? 0.03 : 0.12) * nt, 0.36) * r;
-            double t = (double) per * std::max(std::ceil(wgs / 256) * step, step + 0.6);
-            if (sp > 1) t += (double) sp * out * 8 / 4e6 + 3.0;
-            if (t < best) {
-                best = t;
-                rg = r;
-                splits = (int) sp;
-                ks = (int) per * bk;
-            }
-        }
-}
-
-template <int NT, int RG>
-static void launch_gen(const GemmParams & p, bool wbf, bool xc, float * part, int splits, int64_t batches, int ks,
-                       hipStream_t s) {
-    const int nt_m = (int) ((p.M + 64 * RG - 1) / (64 * RG)), nt_n = (int) ((p.N + 16 * NT - 1) / (16 * NT));
-    const dim3 grid((unsigned) (nt_m * nt_n), (unsigned) splits, (unsigned) batches), block(kGenThreads);
-    if constexpr (NT <= 4) {
-        if (wbf) {
-            if (xc) hipLaunchKernelGGL((gemm_gen<NT, RG, true, true>), grid, block, 0, s, p, part, nt_m, nt_n, ks);
-            else hipLaunchKernelGGL((gemm_gen<NT, RG, true, false>), grid, block, 0, s, p, part, nt_m, nt_n, ks);
-            return;
-        }
-    }
-    if (xc) hipLaunchKernelGGL((gemm_gen<NT, RG, false, true>), grid, block, 0, s, p, part, nt_m, nt_n, ks);
-    else hipLaunchKernelGGL((gemm_gen<NT, RG, false, false>), grid, block, 0, s, p, part, nt_m, nt_n, ks);
-}
-
-// f32 weights, or bf16 weights with at most 64 tokens.
-static hipError_t run_gen(const GemmArgs & a, const GemmParams & p, hipStream_t s) {
-    const bool wbf = a.w_type == WAMX_TYPE_BF16, xbf = a.x_type == WAMX_TYPE_BF16;
-    if (!xbf && a.x_type != WAMX_TYPE_F32) return hipErrorInvalidValue;
-    const int64_t batches = a.B2 * a.B3;
-    // The partials' reduce walks the batches' outputs as one matrix.
-    const bool flat = batches == 1 || (a.epi == WAMX_EPI_NONE && a.ldy == a.M && a.y_bs2 == a.N * a.M &&
-                                       (a.B3 == 1 || a.y_bs3 == a.B2 * a.y_bs2));
-    int nt, rg, splits, ks;
-    gen_plan(p, wbf, batches, flat && a.ws && aligned16(a.ws), a.ws_bytes, nt, rg, splits, ks);
-    float * part = splits > 1 ? (float *) a.ws : nullptr;
-    switch (nt * 2 + rg - 1) {
-        case 2: launch_gen<1, 1>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
-        case 3: launch_gen<1, 2>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
-        case 4: launch_gen<2, 1>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
-        case 5: launch_gen<2, 2>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
-        case 6: launch_gen<3, 1>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
-        case 7: launch_gen<3, 2>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
-        case 8: launch_gen<4, 1>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
-        case 9: launch_gen<4, 2>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
-        default: launch_gen<8, 2>(p, wbf, wbf != xbf, part, splits, batches, ks, s); break;
-    }
-    if (splits > 1) {
-        GemmParams q = p;
-        q.N = p.N * batches;
-        launch_reduce(q, part, splits, s);
-    }
-    return hipGetLastError();
-}
-
 hipError_t launch_partial_sum(const float * part, int splits, int64_t N, int64_t M, void * y, int32_t y_type,
                               int64_t ldy, hipStream_t s) {
     GemmParams p{};
@@ -2447,13 +2355,16 @@ hipError_t launch_gemm(const GemmArgs & a, hipStream_t s) {
     // Tiled weights exist for the few-token products only.
     if (a.w_tiled && (!vec || batches != 1 || a.N > 64 || a.M % 16 != 0 || a.K % 32 != 0))
         return hipErrorNotSupported;
-    if (vec && batches == 1 && a.N <= 64) {
+    if (a.w_tiled) {
         allow_skinny_lds();
-        return run_skinny(p, xf32, a.w_tiled, a.ws, a.ws_bytes, s);
+        return run_skinny(p, xf32, a.ws, a.ws_bytes, s);
     }
-    // Few tokens in batches or with unaligned rows (the tiles below would pad
-    // them to 128 and leave most CUs idle).
-    if (a.N <= 64) return run_gen(a, p, s);
+    // Few tokens (the tiles below would pad them to 128).
+    if (a.N <= 64) {
+        const size_t need = vec && batches == 1 ? skinny_workspace_bytes(a.M, a.N, a.K) : 0;
+        if (need && (!a.ws || need > a.ws_bytes || !aligned16(a.ws))) return hipErrorInvalidValue;
+        return run_gen(a, p, s);
+    }
     if (vec && !xf32 && batches == 1) {
         hipError_t err = hipSuccess;
         if (dispatch_dma(p, a.ws, a.ws_bytes, s, err)) return err;
