@@ -228,7 +228,7 @@ static int64_t es(const wamx_tensor * t) { return (int64_t) wamx_type_size(t->ty
 
 static bool rows_contig(const wamx_tensor * t) { return t->nb[0] == (size_t) es(t); }
 
-static hipError_t run_mul_mat(wamx_backend * be, const wamx_tensor * node) {
+static GemmArgs mul_mat_args(wamx_backend * be, const wamx_tensor * node) {
     const wamx_tensor * a = node->src[0];
     const wamx_tensor * b = node->src[1];
     GemmArgs g;
@@ -257,7 +257,11 @@ static hipError_t run_mul_mat(wamx_backend * be, const wamx_tensor * node) {
     g.ws = be->cws;
     g.ws_bytes = kWorkspaceBytes;
     g.w_tiled = tensor_is_tiled(a);
-    return launch_gemm(g, be->cs);
+    return g;
+}
+
+static hipError_t run_mul_mat(wamx_backend * be, const wamx_tensor * node) {
+    return launch_gemm(mul_mat_args(be, node), be->cs);
 }
 
 static GemmArgs linear_args(wamx_backend * be, const wamx_tensor * node) {
@@ -545,6 +549,126 @@ static int match_f32_fusion(const wamx_backend * be, wamx_cgraph * g, int i, int
         }
     }
     return -1;
+}
+
+// ---------------------------------------------------------------------------
+// Product chains: a 2-D MUL_MAT directly followed by up to kMaxStages
+// element-wise nodes that each read the one before (bias ADD, residual or
+// gated residual, MUL, GELU, bias + GELU), or a bf16 CONV_2D and its bias ADD.
+// The product's last launch applies them, with each node's own rounding, and
+// writes every node's output, so other readers of an intermediate see it as
+// before.  An operand may share memory with a chain output only as the same
+// matrix overwritten in place by its own stage or a later one; the product's
+// inputs with none.
+// ---------------------------------------------------------------------------
+struct Span {
+    const char *b, *e;
+};
+static Span span_of(const wamx_tensor * t) {
+    const char * p = (const char *) t->data;
+    size_t n = wamx_type_size(t->type);
+    for (int i = 0; i < 4; ++i) n += (size_t) (t->ne[i] - 1) * t->nb[i];
+    return Span{p, p + n};
+}
+static bool disjoint(const wamx_tensor * a, const wamx_tensor * b) {
+    const Span x = span_of(a), y = span_of(b);
+    return x.e <= y.b || y.e <= x.b;
+}
+
+// Fills c with the stages after node i; returns the last node they cover (> i)
+// or -1.  placed: the tensors have memory, which is checked; the allocator
+// asks before, and keeps a chain's inputs live through its last node.
+static int match_chain(wamx_cgraph * g, int i, int n, bool lanes, bool placed, Chain & c) {
+    const wamx_tensor * prod = wamx_graph_node(g, i);
+    const bool conv = prod->op == WAMX_OP_CONV_2D;
+    const int32_t typ = prod->type;
+    if (!conv && (prod->op != WAMX_OP_MUL_MAT || (prod->src[0]->type == WAMX_TYPE_BF16 && prod->ne[1] > 64))) return -1;
+    if ((typ != WAMX_TYPE_F32 && typ != WAMX_TYPE_BF16) || !wamx_is_contiguous(prod) || wamx_nelements(prod) <= 0)
+        return -1;
+    if (conv ? typ != WAMX_TYPE_BF16 : prod->ne[2] != 1 || prod->ne[3] != 1) return -1;
+    const wamx_tensor * outs[kMaxStages + 1] = {prod};
+    const wamx_tensor * ops[kMaxStages] = {};
+    const wamx_tensor * cur = prod;
+    int last = -1;
+    c.n = 0;
+    for (int j = next_compute(g, i, n, lanes); j < n && c.n < (conv ? 1 : kMaxStages); j = next_compute(g, j, n, lanes)) {
+        const wamx_tensor * t = wamx_graph_node(g, j);
+        if (t->type != typ || !wamx_are_same_shape(t, prod) || !wamx_is_contiguous(t) || (placed && !t->data)) break;
+        ChainStage st;
+        const wamx_tensor * o = nullptr;     // the operand
+        const wamx_tensor * gate = nullptr;
+        auto row = [&](const wamx_tensor * x, int32_t type) {
+            return x->type == type && x->nb[0] == wamx_type_size(type) && x->ne[0] == prod->ne[0] && x->ne[1] == 1 &&
+                   x->ne[2] == 1 && x->ne[3] == 1;
+        };
+        if (t->op == WAMX_OP_ADD && t->src[2]) {
+            if (t->src[1] != cur || t->src[0] == cur || typ != WAMX_TYPE_BF16) break;
+            o = t->src[0];
+            gate = t->src[2];
+            if (!row(gate, gate->type) || (gate->type != WAMX_TYPE_F32 && gate->type != WAMX_TYPE_BF16)) break;
+            st.kind = kStageGated;
+        } else if (t->op == WAMX_OP_ADD || t->op == WAMX_OP_MUL) {
+            if ((t->src[0] == cur) == (t->src[1] == cur)) break;
+            o = t->src[0] == cur ? t->src[1] : t->src[0];
+            const bool add = t->op == WAMX_OP_ADD;
+            if (conv) {  // bias [1, 1, OC, 1]
+                if (!add || o->type != typ || o->ne[0] != 1 || o->ne[1] != 1 || o->ne[2] != prod->ne[2] ||
+                    o->ne[3] != 1 || (o->ne[2] > 1 && o->nb[2] != 2))
+                    break;
+                st.kind = kStageAddRow;
+            } else {
+                st.kind = row(o, typ) ? (add ? kStageAddRow : kStageMulRow) : add ? kStageAdd : kStageMul;
+            }
+        } else if (t->op == WAMX_OP_UNARY && t->op_params[0] == WAMX_UNARY_GELU) {
+            if (t->src[0] != cur) break;
+            o = t->src[1];
+            if (o && !row(o, typ)) break;
+            st.kind = o ? kStageBiasGelu : kStageGelu;
+        } else {
+            break;
+        }
+        const bool matrix = st.kind == kStageAdd || st.kind == kStageMul || st.kind == kStageGated;
+        if (matrix && (o->type != typ || !wamx_are_same_shape(o, prod) || o->nb[0] != wamx_type_size(typ))) break;
+        if (placed && ((o && !o->data) || (gate && !gate->data))) break;
+        // Memory: this output against the inputs, the operands and the earlier
+        // outputs; this operand against the earlier outputs.
+        bool ok = true;
+        for (int k = 0; placed && k < 2; ++k) ok = ok && disjoint(t, prod->src[k]) && disjoint(prod, prod->src[k]);
+        for (int k = 0; placed && k <= c.n; ++k) {
+            ok = ok && (t->data == outs[k]->data || disjoint(t, outs[k]));
+            if (o) ok = ok && disjoint(o, outs[k]);
+            if (gate) ok = ok && disjoint(gate, outs[k]);
+        }
+        ops[c.n] = o;
+        for (int k = 0; placed && k <= c.n; ++k) {
+            const wamx_tensor * x = ops[k];
+            if (!x || disjoint(t, x)) continue;
+            ok = ok && t->data == x->data && wamx_are_same_shape(t, x) && wamx_is_contiguous(x);
+        }
+        if (placed && gate) ok = ok && disjoint(gate, t);
+        for (int k = 0; placed && k < c.n; ++k)
+            if (c.st[k].gate) ok = ok && ((const char *) c.st[k].gate >= span_of(t).e ||
+                                          (const char *) c.st[k].gate + prod->ne[0] * 4 <= span_of(t).b);
+        if (!ok) break;
+        st.a = o ? o->data : nullptr;
+        st.lda = matrix ? (int64_t) (o->nb[1] / wamx_type_size(typ)) : 0;
+        st.gate = gate ? gate->data : nullptr;
+        st.gate_type = gate ? gate->type : WAMX_TYPE_F32;
+        st.out = t->data;
+        if (c.n > 0 && c.st[c.n - 1].out == t->data) c.st[c.n - 1].out = nullptr;
+        c.st[c.n++] = st;
+        outs[c.n] = t;
+        cur = t;
+        last = j;
+    }
+    return last;
+}
+
+static hipError_t run_chain(wamx_backend * be, const wamx_tensor * node, const Chain & c) {
+    if (node->op == WAMX_OP_CONV_2D)
+        return launch_conv2d(ref_of(node->src[0]), ref_of(node->src[1]), ref_of(node), node->op_params, be->cws,
+                             kWorkspaceBytes, be->cs, c.st[0].a, c.st[0].out);
+    return launch_gemm_chain(mul_mat_args(be, node), c, be->cs);
 }
 
 static hipError_t run_f32_fusion(wamx_backend * be, const F32Fusion & f) {
@@ -1038,6 +1162,39 @@ static wamx_status run_nodes(wamx_backend * be, wamx_cgraph * g) {
                 }
             }
         }
+        if (node->op == WAMX_OP_MUL_MAT || node->op == WAMX_OP_CONV_2D) {
+            Chain c;
+            const int last = match_chain(g, i, n, two, true, c);
+            int dep = -1;
+            if (last > i) {
+                nm = 0;
+                for (int j = i; j <= last && nm < 8; ++j) {
+                    const wamx_tensor * t = wamx_graph_node(g, j);
+                    if (is_noop(t) || (two && (t->lane ? 1 : 0) != lane)) continue;
+                    members[nm++] = j;
+                    dep = std::max(dep, two ? wait_for[j] : -1);
+                }
+            }
+            // As above: a member that must follow a later other-lane node keeps
+            // the nodes apart.
+            if (last > i && dep <= i) {
+                if (dep >= 0) hipStreamWaitEvent(be->cs, be->events[slot[dep]], 0);
+                const hipError_t err = run_chain(be, node, c);
+                if (err == hipSuccess) {
+                    fused = true;
+                    for (int m = 0; m < nm; ++m) done[members[m]] = 1;
+                } else if (err != hipErrorNotSupported) {
+                    set_errorf("graph_compute: node %d (%s '%s') with the nodes after it failed: %s", i,
+                               wamx_op_name(node->op), node->name, hipGetErrorString(err));
+                    status = WAMX_STATUS_FAILED;
+                    break;
+                }
+            }
+            if (!fused) {
+                nm = 1;
+                members[0] = i;
+            }
+        }
         if (!fused && (node->op == WAMX_OP_NORM || node->op == WAMX_OP_MUL)) {
             F32Fusion f;
             const int last = match_f32_fusion(be, g, i, n, f);
@@ -1310,9 +1467,24 @@ static bool gallocr_alloc(wamx_gallocr * ga, wamx_cgraph * g) {
             }
         }
     }
+    bool two = false;
+    for (int i = 0; i < n && !two; ++i) two = wamx_graph_node(g, i)->lane != 0;
+    // Products with the element-wise nodes after them (match_chain).
+    for (int i = 0; i < n; ++i) {
+        wamx_tensor * node = wamx_graph_node(g, i);
+        if (node->op != WAMX_OP_MUL_MAT && node->op != WAMX_OP_CONV_2D) continue;
+        Chain c;
+        const int last = match_chain(g, i, n, two, false, c);
+        for (int j = i; j <= last; ++j) {
+            wamx_tensor * m = wamx_graph_node(g, j);
+            if (j > i && (is_noop(m) || (two && m->lane != node->lane))) continue;
+            for (int k = 0; k < WAMX_MAX_SRC; ++k) {
+                wamx_tensor * r = m->src[k] ? root_of(m->src[k]) : nullptr;
+                if (r && last_use.count(r)) last_use[r] = std::max(last_use[r], last);
+            }
+        }
+    }
     if (ga->be->fuse_rows) {
-        bool two = false;
-        for (int i = 0; i < n && !two; ++i) two = wamx_graph_node(g, i)->lane != 0;
         for (int i = 0; i < n; ++i) {
             wamx_tensor * node = wamx_graph_node(g, i);
             if (node->op != WAMX_OP_LINEAR) continue;

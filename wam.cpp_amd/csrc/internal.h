@@ -66,9 +66,10 @@ constexpr size_t kBackendWorkspaceBytes = 64ull << 20;
 // tokens, given ws_bytes of workspace; 0 when the product takes no K split.
 size_t linear_split_bytes(int64_t M, int64_t N, int64_t K, int32_t x_type, size_t ws_bytes);
 
-// y[n][m] (row stride ldy) = sum over splits of part[split][n][m], in split order.
+// y[n][m] (row stride ldy) = sum over splits of part[split][n][m], in split
+// order; with out: out[n][m] = bf16(y + bias[n]) too (y bf16).
 hipError_t launch_partial_sum(const float * part, int splits, int64_t N, int64_t M, void * y, int32_t y_type,
-                              int64_t ldy, hipStream_t s);
+                              int64_t ldy, hipStream_t s, const void * bias = nullptr, void * out = nullptr);
 
 // Row ops that consume a skinny GEMM's output, applied by its split-K reduce
 // in the same launch (one workgroup per token row).  The GEMM output itself
@@ -118,6 +119,28 @@ struct RowPost {
 // that it splits (the batched denoise step).  Returns hipErrorNotSupported,
 // launching nothing, when the product or the row op does not fit that path.
 hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStream_t s);
+
+// Element-wise nodes that follow a product, applied by the reduce of its K
+// slices: v is the product's value as its node stores it, each stage's result
+// is rounded to the output type, and every node's output is written (but one
+// whose tensor the next stage overwrites in place).
+enum { kStageAddRow = 1, kStageAdd, kStageMulRow, kStageMul, kStageGelu, kStageBiasGelu, kStageGated };
+struct ChainStage {
+    int32_t kind = 0;
+    const void * a = nullptr;      // row [M] or matrix [N][lda], of the output type
+    int64_t lda = 0;
+    const void * gate = nullptr;   // kStageGated: a + v * gate[m], one rounding
+    int32_t gate_type = WAMX_TYPE_F32;
+    void * out = nullptr;          // null: not written
+};
+constexpr int kMaxStages = 3;
+struct Chain {
+    int32_t n = 0;
+    ChainStage st[kMaxStages];
+};
+// The product and its chain; hipErrorNotSupported, launching nothing, where
+// the product is not one that gemm_gen splits along K.
+hipError_t launch_gemm_chain(const GemmArgs & a, const Chain & c, hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Row-wise norms (bf16 / f32), bias+GELU, gated residuals.
@@ -172,8 +195,11 @@ hipError_t launch_im2col(const TensorRef & src, const TensorRef & dst, int KW, i
 // image and kernel packed channels-last at the end of ws, f32 partials before
 // them.  f32: im2col row chunks in the upper half of ws, the GEMM's partials
 // in the lower half.
+// bias (bf16 [OC]) with out: also out = bf16(dst + bias) as the ADD node after
+// a bf16 convolution; hipErrorNotSupported, launching nothing, where the
+// implicit GEMM does not take it.
 hipError_t launch_conv2d(const TensorRef & kernel, const TensorRef & input, const TensorRef & dst, const int32_t * pp,
-                         void * ws, size_t ws_bytes, hipStream_t s);
+                         void * ws, size_t ws_bytes, hipStream_t s, const void * bias = nullptr, void * out = nullptr);
 hipError_t launch_modulation(const void * mod, int32_t mod_type, const void * tables, int32_t tab_type, float * out,
                              int64_t per_layer, int64_t layers, hipStream_t s, int64_t steps = 1);
 // atomicMin of the index of every Inf / NaN of p[0, n) into *first (n < 2^32).

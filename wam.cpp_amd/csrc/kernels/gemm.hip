@@ -1191,6 +1191,78 @@ __global__ __launch_bounds__(256) void gemm_skinny_reduce(GemmParams p, const fl
     for (int e = 0; e < V; ++e) store_pre(p, p.y, n, m + e, s[e], bias[e], res[e], gate[e]);
 }
 
+// The reduce of a product and the element-wise nodes after it (Chain), four
+// outputs of a row per thread, every operand requested before the first
+// partial is summed.  BF: bf16 outputs and operands, else f32.  Each node as a
+// launch of its own took 4.5 us at 48 x 3072, where the chain adds nothing to
+// the reduce's 4.8.
+template <bool BF>
+__global__ __launch_bounds__(256) void gemm_reduce_chain(GemmParams p, Chain c, const float * __restrict__ part,
+                                                         int splits) {
+    const int64_t total = p.N * p.M, i0 = ((int64_t) blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i0 >= total) return;
+    const int64_t n = i0 / p.M, m = i0 % p.M;
+    auto load4 = [](const void * base, int64_t i, bool bf, float (&o)[4]) {
+        if (bf) {
+            const uint2 u = *(const uint2 *) ((const uint16_t *) base + i);
+            o[0] = __uint_as_float(u.x << 16), o[1] = __uint_as_float(u.x & 0xFFFF0000u);
+            o[2] = __uint_as_float(u.y << 16), o[3] = __uint_as_float(u.y & 0xFFFF0000u);
+        } else {
+            const float4 v = *(const float4 *) ((const float *) base + i);
+            o[0] = v.x, o[1] = v.y, o[2] = v.z, o[3] = v.w;
+        }
+    };
+    float a[kMaxStages][4] = {}, g[kMaxStages][4] = {};
+#pragma unroll
+    for (int k = 0; k < kMaxStages; ++k) {
+        const ChainStage & st = c.st[k];
+        if (k >= c.n || st.kind == kStageGelu) continue;
+        const bool row = st.kind == kStageAddRow || st.kind == kStageMulRow || st.kind == kStageBiasGelu;
+        load4(st.a, row ? m : n * st.lda + m, BF, a[k]);
+        if (st.kind == kStageGated) load4(st.gate, m, st.gate_type == WAMX_TYPE_BF16, g[k]);
+    }
+    f32x4_t s = *(const f32x4_t *) (part + i0);
+    constexpr int kBatch = 8;
+    for (int sp0 = 1; sp0 < splits; sp0 += kBatch) {
+        f32x4_t v[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+            if (sp0 + u < splits) v[u] = *(const f32x4_t *) (part + (int64_t) (sp0 + u) * total + i0);
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+            if (sp0 + u < splits) s += v[u];
+    }
+    float v[4];
+    auto put = [&](void * out, int64_t i) {
+        if (BF) *(uint2 *) ((uint16_t *) out + i) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        else *(float4 *) ((float *) out + i) = make_float4(v[0], v[1], v[2], v[3]);
+    };
+    auto round_v = [&]() {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = BF ? round_bf16(v[e]) : v[e];
+    };
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = s[e];
+    round_v();
+    if (p.y) put(p.y, n * p.ldy + m);
+#pragma unroll
+    for (int k = 0; k < kMaxStages; ++k) {
+        if (k >= c.n) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) switch (c.st[k].kind) {  // the nodes' own rounding: no contraction across them
+            case kStageAddRow:
+            case kStageAdd: v[e] = __fadd_rn(v[e], a[k][e]); break;
+            case kStageMulRow:
+            case kStageMul: v[e] = __fmul_rn(v[e], a[k][e]); break;
+            case kStageGelu: v[e] = gelu_tanh(v[e]); break;
+            case kStageBiasGelu: v[e] = gelu_tanh(__fadd_rn(v[e], a[k][e])); break;
+            default: v[e] = fmaf(v[e], g[k][e], a[k][e]); break;
+        }
+        round_v();
+        if (c.st[k].out) put(c.st[k].out, n * p.M + m);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // skinny_reduce_row: the split-K reduce of one token row fused with the row op
 // that consumes the GEMM output, so a denoise-step projection costs two
@@ -2328,8 +2400,50 @@ __global__ void round_rows_bf16_kernel(const float * __restrict__ x, int64_t ldx
     *(uint4 *) (y + r * K + 8 * c) = pack8(v);
 }
 
+hipError_t launch_gemm_chain(const GemmArgs & a, const Chain & c, hipStream_t s) {
+    GemmParams p = make_params(a);
+    const bool wbf = a.w_type == WAMX_TYPE_BF16, xbf = a.x_type == WAMX_TYPE_BF16, bf = a.y_type == WAMX_TYPE_BF16;
+    if (a.B2 * a.B3 != 1 || a.M <= 0 || a.N <= 0 || a.K <= 0 || a.w_tiled || a.epi != WAMX_EPI_NONE || c.n < 1 ||
+        c.n > kMaxStages || (!wbf && a.w_type != WAMX_TYPE_F32) || (!xbf && a.x_type != WAMX_TYPE_F32) ||
+        (wbf && a.N > 64) || a.M % 4 != 0 || a.ldy % 4 != 0 || !a.ws || !aligned16(a.ws) ||
+        (wbf && skinny_workspace_bytes(a.M, a.N, a.K) > a.ws_bytes))
+        return hipErrorNotSupported;
+    auto aligned = [&](const void * q) { return ((uintptr_t) q & (bf ? 7 : 15)) == 0; };
+    if (!aligned(a.y)) return hipErrorNotSupported;
+    for (int k = 0; k < c.n; ++k)
+        if (!aligned(c.st[k].a) || !aligned(c.st[k].out) || c.st[k].lda % 4 != 0 || !aligned16(c.st[k].gate))
+            return hipErrorNotSupported;
+    const GenPlan b = gen_plan(p, wbf, xbf, 1, a.ws_bytes);
+    if (b.splits <= 1) return hipErrorNotSupported;
+    launch_gen_part(p, wbf, xbf, (float *) a.ws, b, 1, s);
+    const dim3 grid((unsigned) ((p.N * p.M / 4 + 255) / 256));
+    if (bf) hipLaunchKernelGGL(gemm_reduce_chain<true>, grid, dim3(256), 0, s, p, c, (const float *) a.ws, b.splits);
+    else hipLaunchKernelGGL(gemm_reduce_chain<false>, grid, dim3(256), 0, s, p, c, (const float *) a.ws, b.splits);
+    return hipGetLastError();
+}
+
+__global__ __launch_bounds__(256) void partial_sum_bias(const float * __restrict__ part, int splits, int64_t N,
+                                                        int64_t M, uint16_t * __restrict__ y,
+                                                        uint16_t * __restrict__ out, int64_t ldy,
+                                                        const uint16_t * __restrict__ bias) {
+    const int64_t total = N * M, i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+    if (i >= total) return;
+    const int64_t n = i / M, m = i % M;
+    float s = part[i];
+    for (int sp = 1; sp < splits; ++sp) s += part[sp * total + i];
+    const float v = round_bf16(s);
+    y[n * ldy + m] = f32_to_bf16(s);
+    out[n * ldy + m] = f32_to_bf16(v + bf16_to_f32(bias[n]));
+}
+
 hipError_t launch_partial_sum(const float * part, int splits, int64_t N, int64_t M, void * y, int32_t y_type,
-                              int64_t ldy, hipStream_t s) {
+                              int64_t ldy, hipStream_t s, const void * bias, void * out) {
+    if (out) {
+        if (y_type != WAMX_TYPE_BF16) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(partial_sum_bias, dim3((unsigned) ((N * M + 255) / 256)), dim3(256), 0, s, part, splits, N,
+                           M, (uint16_t *) y, (uint16_t *) out, ldy, (const uint16_t *) bias);
+        return hipGetLastError();
+    }
     GemmParams p{};
     p.y = y;
     p.y_type = y_type;

@@ -140,6 +140,8 @@ struct ConvGemm {
     uint16_t * xp;        // [rows][IWp][ICp], padded image rows from row iy0
     uint16_t * kp;        // [OC][taps][ICp]
     uint16_t * y;         // image b [OC][P], at the band's first pixel
+    uint16_t * out;       // y + bias (laid out as y), or null
+    const uint16_t * bias;
     float * part;         // [splits][OC][P of the band], or null
     int64_t IW, IH, IC, OC, P;       // P: pixels of a whole output plane (row stride of y)
     int IWp, ICp, OW, pix;           // pix: output pixels of the band
@@ -333,7 +335,10 @@ __global__ __launch_bounds__(512) void conv_gemm_kernel(ConvGemm c) {
                     const int64_t oc = ob + 16 * i + v, p = pb + 16 * j;
                     if (!decltype(all)::value && (oc >= c.OC || p >= c.pix)) continue;
                     if (c.part) c.part[((int64_t) blockIdx.y * c.OC + oc) * c.pix + p] = acc[i][j][v];
-                    else c.y[oc * c.P + p] = f32_to_bf16(acc[i][j][v]);
+                    else {
+                        c.y[oc * c.P + p] = f32_to_bf16(acc[i][j][v]);
+                        if (c.out) c.out[oc * c.P + p] = f32_to_bf16(round_bf16(acc[i][j][v]) + bf16_to_f32(c.bias[oc]));
+                    }
                 }
     };
     if (whole) store(std::true_type{});
@@ -342,8 +347,8 @@ __global__ __launch_bounds__(512) void conv_gemm_kernel(ConvGemm c) {
 
 // Returns hipErrorNotSupported, launching nothing, when not even one output
 // row's image rows fit the workspace beside the packed kernel.
-static hipError_t conv_implicit(const ConvDev & d, const void * kernel, void * dst, int64_t OC, int64_t B, void * ws,
-                                size_t ws_bytes, hipStream_t s) {
+static hipError_t conv_implicit(const ConvDev & d, const void * kernel, void * dst, const void * bias, void * out,
+                                int64_t OC, int64_t B, void * ws, size_t ws_bytes, hipStream_t s) {
     ConvGemm c{};
     c.IW = d.IW, c.IH = d.IH, c.IC = d.IC, c.OC = OC, c.P = d.OW * d.OH;
     c.k = (const uint16_t *) kernel;
@@ -369,6 +374,8 @@ static hipError_t conv_implicit(const ConvDev & d, const void * kernel, void * d
             const int64_t n = std::min(band, d.OH - oy);
             c.x = (const uint16_t *) d.x + b * d.IC * d.IH * d.IW;
             c.y = (uint16_t *) dst + b * OC * c.P + oy * d.OW;
+            c.out = out ? (uint16_t *) out + b * OC * c.P + oy * d.OW : nullptr;
+            c.bias = (const uint16_t *) bias;
             c.iy0 = (int) (oy * d.s1), c.rows = (int) ((n - 1) * d.s1 + reach), c.pix = (int) (n * d.OW);
             c.xp = (uint16_t *) ((char *) c.kp - (((size_t) c.rows * row + 255) / 256 * 256));
             const int image = (int) ((IWp + kPackPix - 1) / kPackPix * (ICp / 32) * c.rows);
@@ -393,7 +400,7 @@ static hipError_t conv_implicit(const ConvDev & d, const void * kernel, void * d
             }
             if (splits > 1) {
                 const hipError_t e = launch_partial_sum((const float *) ws, (int) splits, OC, c.pix, c.y,
-                                                        WAMX_TYPE_BF16, c.P, s);
+                                                        WAMX_TYPE_BF16, c.P, s, c.bias, c.out);
                 if (e != hipSuccess) return e;
             }
         }
@@ -401,7 +408,7 @@ static hipError_t conv_implicit(const ConvDev & d, const void * kernel, void * d
 }
 
 hipError_t launch_conv2d(const TensorRef & kernel, const TensorRef & input, const TensorRef & dst, const int32_t * pp,
-                         void * ws, size_t ws_bytes, hipStream_t s) {
+                         void * ws, size_t ws_bytes, hipStream_t s, const void * bias, void * out) {
     const bool bf = kernel.type == WAMX_TYPE_BF16;
     if ((bf && (input.type != WAMX_TYPE_BF16 || dst.type != WAMX_TYPE_BF16)) ||
         (!bf && (kernel.type != WAMX_TYPE_F32 || input.type != WAMX_TYPE_F32 || dst.type != WAMX_TYPE_F32)))
@@ -426,9 +433,10 @@ hipError_t launch_conv2d(const TensorRef & kernel, const TensorRef & input, cons
     const int64_t K = c.IC * c.KH * c.KW, P = c.OW * c.OH, OC = kernel.ne[3], B = input.ne[3];
     const size_t es = bf ? 2 : 4;
     if (bf) {
-        const hipError_t e = conv_implicit(c, kernel.data, dst.data, OC, B, ws, ws_bytes, s);
+        const hipError_t e = conv_implicit(c, kernel.data, dst.data, bias, out, OC, B, ws, ws_bytes, s);
         if (e != hipErrorNotSupported) return e;
     }
+    if (out) return hipErrorNotSupported;
     // f32, and images of which not one band fits the workspace: column matrix.
     // Upper workspace half: the column chunk; lower half: the GEMM's split-K partials.
     const size_t half = ws_bytes / 2 / 256 * 256;
