@@ -532,3 +532,19 @@ def test_empty_and_refused_sizes(wx, be):
                               128) != 0
     be.sync()
     assert np.array_equal(y.download(np.uint16, (4096,)), sentinel)
+
+
+# The K-sliced 256 x 256 and 192 x 192 tiles (dma_plan), whole and with ragged
+# edges, and their f32 outputs.
+@pytest.mark.parametrize("M,N,K", [(3072, 2048, 14336), (3072, 1000, 14336), (3000, 500, 14336), (14336, 1000, 512),
+                                   (9216, 1030, 256), (4096, 1500, 4096)])
+@pytest.mark.parametrize("xt", ["f32", "bf16"])
+def test_mul_mat_sliced_large_tiles_integers_exact(wx, be, M, N, K, xt):
+    print(f"mul_mat sliced large tiles M={M} N={N} K={K} x={xt}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    w = rng.integers(-4, 5, (M, K)).astype(np.float32)
+    x = rng.integers(-4, 5, (N, K)).astype(np.float32)
+    ref = x @ w.T  # exact in f32: sums below 2^24
+    xin = x if xt == "f32" else bf16(x)
+    assert np.array_equal(gpu_mul_mat(wx, be, bf16(w), xin, wx.TYPE_F32), ref)
+    assert np.array_equal(gpu_mul_mat(wx, be, bf16(w), xin, wx.TYPE_BF16), bf16(ref))

@@ -788,7 +788,10 @@ __global__ __launch_bounds__(64 * WM * WN * (SCHED == kSchedProducer ? 2 : 1), 1
         if (i * RPI < BM) soff[i] = (uint32_t) ((min(n0 + r, N - 1) * p.ldx + 8 * c) * 2);
         else soff[i] = (uint32_t) ((min(m0 + min(r - BM, BN - 1), M - 1) * p.ldw + 8 * c) * 2);
     }
-    const char * const xb = (const char *) p.x, * const wb = (const char *) p.w;
+    // K slices along blockIdx.y (launch_pipe_splitk): p.K columns each, into
+    // f32 partial planes.
+    const int64_t slice = blockIdx.y;
+    const char * const xb = (const char *) p.x + slice * p.K * 2, * const wb = (const char *) p.w + slice * p.K * 2;
     uint16_t * const stp[5] = {st0, st1, st2, S > 3 ? st3 : st0, S > 4 ? st4 : st0};
     auto dma = [&](int kt, int stage) {
         const uint32_t koff = (uint32_t) min(kt, nk - 1) * BK * 2;
@@ -981,6 +984,12 @@ __global__ __launch_bounds__(64 * WM * WN * (SCHED == kSchedProducer ? 2 : 1), 1
     constexpr int REG = 32 * (C::kWaveN + 8), WPS = E / REG;
     static_assert(WPS >= 1 && WPS * S >= C::kWaves, "staging regions must fit in the ring");
     __syncthreads();
+    if constexpr (MF == 32) {
+        if (p.y_type == WAMX_TYPE_F32) {
+            tile_store<kEpiF32>(p, (char *) p.y + slice * p.N * p.M * 4, nullptr, acc, nb, mb, lane);
+            return;
+        }
+    }
     const int sa = wave / WPS;
     uint16_t * region = (sa == 0 ? st0 : sa == 1 ? st1 : sa == 2 ? st2 : sa == 3 ? stp[3] : stp[4]) + (wave % WPS) * REG;
     uint16_t * y = (uint16_t *) p.y;
@@ -1961,9 +1970,9 @@ static hipError_t run_dma(const GemmParams & p, hipStream_t s) {
     return hipGetLastError();
 }
 // The pipelined kernel addresses its copies by 32-bit offsets and stores bf16
-// rows in 16-byte chunks.
+// rows in 16-byte chunks, or f32 (32x32 fragments only).
 static bool pipe_ok(const GemmParams & p) {
-    return p.vec_out && (uint64_t) p.N * p.ldx * 2 < (1ull << 32) && (uint64_t) p.M * p.ldw * 2 < (1ull << 32);
+    return (p.vec_out || epi_kind(p) == kEpiF32) && (uint64_t) p.N * p.ldx * 2 < (1ull << 32) && (uint64_t) p.M * p.ldw * 2 < (1ull << 32);
 }
 template <int BM, int BN, int WM, int WN, int S, int SCHED, int BKP, int MF = 32>
 static hipError_t launch_dma_pipe(const GemmParams & p, hipStream_t s) {
@@ -1978,6 +1987,25 @@ template <int BM, int BN, int WM, int WN, int S, int BKF, int SF, int SCHED = kS
 static hipError_t run_dma_pipe(const GemmParams & p, hipStream_t s) {
     if (!pipe_ok(p)) return run_dma<BM, BN, WM, WN, BKF, SF>(p, s);
     return launch_dma_pipe<BM, BN, WM, WN, S, SCHED, BKP>(p, s);
+}
+
+// K slices of the pipelined kernel into f32 partial planes of ws, each of
+// p.K / splits columns, then the reduce with the epilogue.
+template <int BM, int BN, int WM, int WN, int S, int SCHED, int BKP>
+static hipError_t launch_pipe_splitk(const GemmParams & p, int splits, void * ws, hipStream_t s) {
+    GemmParams q = p;
+    q.K = p.K / splits;
+    q.y = ws;
+    q.y_type = WAMX_TYPE_F32;
+    q.ldy = p.M;
+    q.epi = WAMX_EPI_NONE;
+    q.vec_out = 0;
+    const int nt_m = (int) ((p.M + BN - 1) / BN), nt_n = (int) ((p.N + BM - 1) / BM);
+    const int threads = 64 * WM * WN * (SCHED == kSchedProducer ? 2 : 1);
+    hipLaunchKernelGGL((gemm_dma_pipe<BM, BN, WM, WN, S, SCHED, BKP>), dim3((unsigned) (nt_m * nt_n), (unsigned) splits),
+                       dim3(threads), 0, s, q, nt_m, nt_n);
+    launch_reduce(p, (const float *) ws, splits, s);
+    return hipGetLastError();
 }
 
 static int64_t tiles_of(const GemmParams & p, int bm, int bn) { return ((p.N + bm - 1) / bm) * ((p.M + bn - 1) / bn); }
@@ -2058,13 +2086,12 @@ static hipError_t run_dma_splitk(const GemmParams & p, int splits, void * ws, hi
 //    256 x 224 with 16x16 fragments instead where its whole rounds finish
 //    sooner (prefer_tile224: FFN-up 14336 x 3072 in 768 tiles, 3 rounds,
 //    against 672; QKV 9216 x 3072 in 504 against 432), same bits;
-//  * 192 x 192, 4 waves: 3072 x 3072 products, which it cuts into exactly 256
-//    tiles (256 x 256 leaves 112 CUs idle), pipelined with BK 64 and 3
-//    stages, copies issued by 4 producer waves (2-4% faster on O and
-//    FFN-down than without them);
-//  (f32 or unaligned outputs take gemm_dma with BK 32 / 64 and 3 stages);
-//  * 128 x 128, BK 64, 2 stages, 4 waves, two workgroups per CU: small grids
-//    (512-token prompt projections).
+//  * below that dma_plan's choice of 256 x 256, of 192 x 192 (3072 x 3072
+//    products, which it cuts into exactly 256 tiles; pipelined with BK 64 and
+//    3 stages, copies issued by 4 producer waves, 2-4% faster on O and FFN-down
+//    than without them) and of 128 x 128 (BK 64, 2 stages, 4 waves, two
+//    workgroups per CU), in K slices where the tiles leave CUs idle;
+//  (unaligned outputs take gemm_dma with BK 32 / 64 and 3 stages).
 // Returns false when the shape does not meet the path's preconditions.
 static bool tile224_enabled() {
     static const bool on = [] {
@@ -2084,27 +2111,75 @@ static bool prefer_tile224(const GemmParams & p) {
     return 7 * r224 < 8 * r256;
 }
 
+// Tile and K slices below one 256 x 256 tile per CU, by modelled time in us:
+// rounds of one workgroup per CU (two of the 128 x 128 tiles), each K column of
+// a round at the tile's measured rate (a fuller grid runs at a lower clock),
+// the ring's fill and the epilogue, and for slices the planes' traffic and the
+// reduce launch.  The 128 x 128 tiles take dma_splitk_plan's slices.
+//
+// Sweep of tile and slices (us, bf16, weights from HBM): 3072 x 2048 x 14336
+// 191 in two slices of 256 x 256 tiles (192 workgroups) against 226 on 192 x
+// 192 and 255 on 128 x 128; 3072 x 1024 x 14336 113 in four against 144 (128 x
+// 128 in two); 14336 x 1024 x 3072 87 on 224 tiles of 256 x 256 against 120 on
+// 192 x 192; 9216 x 1024 x 3072 80 against 104; 3072 x 512 x 3072 32 on 128 x
+// 128 in four slices against 33 and 36.
+struct DmaPlan {
+    int tile, splits;
+};
+static DmaPlan dma_plan(const GemmParams & p, size_t ws_bytes) {
+    DmaPlan best{128, dma_splitk_plan(p, ws_bytes)};
+    if (!pipe_ok(p)) {
+        if (tiles_of(p, 192, 192) >= 192) best = DmaPlan{192, 1};
+        return best;
+    }
+    auto slices = [&](int sp) {
+        return sp > 1 ? 3.0 + (double) sp * (double) p.N * (double) p.M * 8 / 6e6 : 0.0;
+    };
+    const double k = (double) p.K;
+    const int64_t w = tiles_of(p, 128, 128) * best.splits;
+    double t = 5.0 + (w <= 256 ? 0.0155 : 0.018 * (double) ((w + 511) / 512)) * k / best.splits + slices(best.splits);
+    for (int tile : {192, 256}) {
+        const int64_t tiles = tiles_of(p, tile, tile);
+        for (int sp = 1; sp <= 16; ++sp) {
+            if (p.K % (64 * sp) != 0 || (sp > 1 && (p.K / sp < 256 || (double) sp * p.N * p.M * 4 > (double) ws_bytes)))
+                continue;
+            const int64_t n = tiles * sp;
+            const double rate = tile == 192 ? (n <= 200 ? 0.0165 : 0.0178) : (n <= 200 ? 0.0246 : 0.027);
+            const double u = 8.0 + (double) ((n + 255) / 256) * rate * k / sp + slices(sp);
+            if (u < t) {
+                t = u;
+                best = DmaPlan{tile, sp};
+            }
+        }
+    }
+    return best;
+}
+
 static bool dispatch_dma(const GemmParams & p, void * ws, size_t ws_bytes, hipStream_t s, hipError_t & err) {
     if (p.K % 32 != 0) return false;
     if (tiles_of(p, 256, 256) >= 256) {
         // 256 x 224: FFN-up (14336 features x 3072 tokens) takes 768 tiles,
         // three whole rounds of 256 CUs, where 256 x 256 leaves 672 (2.6).
-        if (pipe_ok(p) && prefer_tile224(p))
+        if (pipe_ok(p) && p.vec_out && prefer_tile224(p))
             err = launch_dma_pipe<256, 224, 4, 2, 4, kSchedPingPong, 32, 16>(p, s);
         else
             err = run_dma_pipe<256, 256, 4, 2, 4, 32, 3, kSchedPingPong>(p, s);
         return true;
     }
     if (p.K % 64 != 0) return false;
-    if (tiles_of(p, 192, 192) >= 192) {
+    if (!ws || ((uintptr_t) ws & 15)) ws_bytes = 0;
+    const DmaPlan d = dma_plan(p, ws_bytes);
+    if (d.tile == 256)
+        err = d.splits > 1 ? launch_pipe_splitk<256, 256, 4, 2, 4, kSchedPingPong, 32>(p, d.splits, ws, s)
+                           : run_dma_pipe<256, 256, 4, 2, 4, 32, 3, kSchedPingPong>(p, s);
+    else if (d.tile == 192)
         // K steps of 64 in a 3-stage ring (144 KB): half the barriers and
         // waits per K of the 4-stage BK 32 ring, same bits.  3072^2 55.6
         // against 64.0 us, FFN-down (K 14336) 234 against 280.
-        err = run_dma_pipe<192, 192, 2, 2, 3, 64, 3, kSchedProducer, 64>(p, s);
-        return true;
-    }
-    const int splits = ws && ((uintptr_t) ws & 15) == 0 ? dma_splitk_plan(p, ws_bytes) : 1;
-    err = splits > 1 ? run_dma_splitk(p, splits, ws, s) : run_dma<128, 128, 2, 2, 64, 2>(p, s);
+        err = d.splits > 1 ? launch_pipe_splitk<192, 192, 2, 2, 3, kSchedProducer, 64>(p, d.splits, ws, s)
+                           : run_dma_pipe<192, 192, 2, 2, 3, 64, 3, kSchedProducer, 64>(p, s);
+    else
+        err = d.splits > 1 ? run_dma_splitk(p, d.splits, ws, s) : run_dma<128, 128, 2, 2, 64, 2>(p, s);
     return true;
 }
 

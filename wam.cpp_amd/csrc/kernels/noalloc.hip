@@ -1,14 +1,15 @@
 // wamx_op_linear_noalloc: wamx_op_linear for callers that cannot allocate
 // device memory (code under HIP graph capture, tight serving loops, hosts
 // that forbid hipMalloc).  The split-K partials of any product that takes a
-// K split (few-token products on the skinny path, and 65..~500-token
-// products on small grids, K-sliced 128 x 128 tiles) live in `scratch`, a
-// file-scope device array of kScratchBytes that every GPU the library runs on
-// holds until the process ends.  Nothing here allocates: no backend is
+// K split (few-token products, and products of more tokens whose tiles leave
+// CUs idle) live in `scratch`, a file-scope device array as large as a
+// backend's workspace that every GPU the library runs on holds until the
+// process ends.  Nothing here allocates: no backend is
 // created, no workspace is malloc'd; the caller passes its stream, inputs and
 // output.  The split is planned as wamx_op_linear plans it with a backend's
-// workspace; a product whose partials would then not fit the array is
-// refused, so both entry points always take the same slices (same bits).
+// workspace, so both entry points always take the same slices (same bits).
+// Products whose split-K partials would pass kSplitLimit by linear_split_bytes
+// are refused.
 //
 // Every call on a GPU shares that GPU's array and it keeps the last call's
 // contents.  The partials are written whole by the part kernel before the
@@ -21,7 +22,8 @@
 
 namespace wamx {
 
-constexpr size_t kScratchBytes = 32ull << 20;   // 32 MiB per GPU
+constexpr size_t kScratchBytes = kBackendWorkspaceBytes;  // per GPU
+constexpr size_t kSplitLimit = 32ull << 20;
 constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -62,10 +64,10 @@ extern "C" wamx_status wamx_op_linear_noalloc(void * stream, const void * w, con
                  "wamx_op_linear_noalloc: residual required");
     WAMX_REQUIRE(epilogue != WAMX_EPI_BIAS_GATED || gate, "wamx_op_linear_noalloc: gate required");
     const size_t need = linear_split_bytes(M, N, K, x_type, kBackendWorkspaceBytes);
-    WAMX_REQUIRE(need <= kScratchBytes,
+    WAMX_REQUIRE(need <= kSplitLimit,
                  "wamx_op_linear_noalloc: a %lld x %lld x %lld product needs %zu bytes of split-K scratch, more than "
                  "the %zu this entry point holds; use wamx_op_linear",
-                 (long long) N, (long long) M, (long long) K, need, kScratchBytes);
+                 (long long) N, (long long) M, (long long) K, need, kSplitLimit);
     void * ws = nullptr;
     WAMX_HIP_TRY(scratch_ptr(&ws));
     GemmArgs g;
