@@ -548,3 +548,20 @@ def test_mul_mat_sliced_large_tiles_integers_exact(wx, be, M, N, K, xt):
     xin = x if xt == "f32" else bf16(x)
     assert np.array_equal(gpu_mul_mat(wx, be, bf16(w), xin, wx.TYPE_F32), ref)
     assert np.array_equal(gpu_mul_mat(wx, be, bf16(w), xin, wx.TYPE_BF16), bf16(ref))
+
+
+# One launch for few tokens (gemm_row16): K below, at and past a round of the
+# waves' 32-column tiles and not a multiple of 32 (row-major), features below
+# and past 16, 1 to 48 tokens, both weight layouts and activation types.
+@pytest.mark.parametrize("M,N,K", [(3072, 1, 3072), (1024, 48, 1024), (16, 17, 32), (40, 5, 72), (1000, 33, 264),
+                                   (2000, 16, 1048), (4096, 32, 2048), (8, 48, 2056)])
+@pytest.mark.parametrize("xt", ["f32", "bf16"])
+def test_few_tokens_one_launch_integers_exact(wx, be, M, N, K, xt):
+    print(f"one-launch mul_mat M={M} N={N} K={K} x={xt}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    w = rng.integers(-4, 5, (M, K)).astype(np.float32)
+    x = rng.integers(-4, 5, (N, K)).astype(np.float32)
+    ref = x @ w.T
+    xin = x if xt == "f32" else bf16(x)
+    assert np.array_equal(gpu_mul_mat(wx, be, bf16(w), xin, wx.TYPE_F32), ref)
+    assert np.array_equal(gpu_mul_mat(wx, be, bf16(w), xin, wx.TYPE_BF16), bf16(ref))

@@ -120,8 +120,7 @@ struct RowPost {
 // launching nothing, when the product or the row op does not fit that path.
 hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStream_t s);
 
-// Element-wise nodes that follow a product, applied by the reduce of its K
-// slices: v is the product's value as its node stores it, each stage's result
+// Element-wise nodes that follow a product, applied by its last launch: v is the product's value as its node stores it, each stage's result
 // is rounded to the output type, and every node's output is written (but one
 // whose tensor the next stage overwrites in place).
 enum { kStageAddRow = 1, kStageAdd, kStageMulRow, kStageMul, kStageGelu, kStageBiasGelu, kStageGated };
@@ -139,7 +138,7 @@ struct Chain {
     ChainStage st[kMaxStages];
 };
 // The product and its chain; hipErrorNotSupported, launching nothing, where
-// the product is not one that gemm_gen splits along K.
+// the product is neither gemm_row16's nor one that gemm_gen splits along K.
 hipError_t launch_gemm_chain(const GemmArgs & a, const Chain & c, hipStream_t s);
 
 // ---------------------------------------------------------------------------

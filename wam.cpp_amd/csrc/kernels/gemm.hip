@@ -12,6 +12,7 @@
 //  * gemm_skinny_tiled, gemm_skinny_wk — N <= 64 tokens (the 48-token action
 //                  expert) on tiled weights: HBM-bound weight streaming with
 //                  MFMA 16x16x32.
+//  * gemm_row16  — few tokens and a modest weight, either layout, one launch.
 //  * gemm_gen    — N <= 64 tokens on row-major weights, batches and any
 //                  alignment included, and f32 weights (the f32 reference
 //                  profile, generic MUL_MAT) on f32 MFMA 16x16x4.
@@ -1940,6 +1941,120 @@ __global__ __launch_bounds__(kGenThreads, 2) void gemm_gen(GemmParams p, float *
 }
 
 // ---------------------------------------------------------------------------
+// gemm_row16: few tokens, one launch.  A workgroup of 8 waves takes 16 features
+// over all of K: wave w multiplies the 32-column k-tiles w, w + 8, ..., so the
+// waves together read 512 adjacent bytes of each weight row (or 8 adjacent 1 KB
+// tiles of the tiled layout), straight into MFMA 16x16x32 operands, U tiles of
+// the wave in flight.  The activations come straight from L2.  The waves' sums
+// meet in LDS in wave order and the epilogue follows, so there are no partials
+// and no reduce launch: what bounds a product of 19 MB at one token is its two
+// launches, not the weights.
+// ---------------------------------------------------------------------------
+constexpr int kRowWaves = 8;
+
+// One output of a product and its chain (gemm_reduce_chain's arithmetic).
+__device__ __forceinline__ void store_chain(const GemmParams & p, const Chain & c, int64_t n, int64_t m, float acc) {
+    const bool bf = p.y_type == WAMX_TYPE_BF16;
+    auto load = [&](const void * a, int64_t i, bool b) {
+        return b ? bf16_to_f32(((const uint16_t *) a)[i]) : ((const float *) a)[i];
+    };
+    auto put = [&](void * out, int64_t i, float v) {
+        if (bf) ((uint16_t *) out)[i] = f32_to_bf16(v);
+        else ((float *) out)[i] = v;
+    };
+    float a[kMaxStages] = {}, g[kMaxStages] = {};
+#pragma unroll
+    for (int k = 0; k < kMaxStages; ++k) {
+        const ChainStage & st = c.st[k];
+        if (k >= c.n || st.kind == kStageGelu) continue;
+        const bool row = st.kind == kStageAddRow || st.kind == kStageMulRow || st.kind == kStageBiasGelu;
+        a[k] = load(st.a, row ? m : n * st.lda + m, bf);
+        if (st.kind == kStageGated) g[k] = load(st.gate, m, st.gate_type == WAMX_TYPE_BF16);
+    }
+    float v = bf ? round_bf16(acc) : acc;
+    put(p.y, n * p.ldy + m, v);
+#pragma unroll
+    for (int k = 0; k < kMaxStages; ++k) {
+        if (k >= c.n) continue;
+        switch (c.st[k].kind) {
+            case kStageAddRow:
+            case kStageAdd: v = __fadd_rn(v, a[k]); break;
+            case kStageMulRow:
+            case kStageMul: v = __fmul_rn(v, a[k]); break;
+            case kStageGelu: v = gelu_tanh(v); break;
+            case kStageBiasGelu: v = gelu_tanh(__fadd_rn(v, a[k])); break;
+            default: v = fmaf(v, g[k], a[k]); break;
+        }
+        if (bf) v = round_bf16(v);
+        if (c.st[k].out) put(c.st[k].out, n * p.M + m, v);
+    }
+}
+
+template <int NT, bool XF32, bool TILED>
+__global__ __launch_bounds__(kRowWaves * 64) void gemm_row16(GemmParams p, Chain c) {
+    constexpr int U = NT == 1 ? 8 : 4;
+    __shared__ float red[kRowWaves][16 * NT][17];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 4, r16 = lane & 15;
+    const int64_t m0 = (int64_t) blockIdx.x * 16;
+    const int K = (int) p.K, tiles = (K + 31) / 32;
+    const uint16_t * w = TILED ? p.w + (m0 / 16) * tiles * 512 + lane * 8 : p.w + min(m0 + r16, p.M - 1) * p.ldw + 8 * g;
+    constexpr int XS = XF32 ? 4 : 2;
+    const char * x[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) x[t] = (const char *) p.x + (min((int64_t) (16 * t + r16), p.N - 1) * p.ldx + 8 * g) * XS;
+    f32x4_t acc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int t0 = wave; t0 < tiles; t0 += kRowWaves * U) {
+        uint4 wv[U], xv[U][NT], xw[XF32 ? U : 1][NT];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            // Past the end the lane's last chunk again, masked below.
+            const int q = min(t0 + u * kRowWaves, tiles - 1), k = min(32 * q, K - 8 - 8 * g);
+            wv[u] = *(const uint4 *) (w + (TILED ? (int64_t) q * 512 : (int64_t) k));
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                xv[u][t] = *(const uint4 *) (x[t] + (int64_t) k * XS);
+                if constexpr (XF32) xw[u][t] = *(const uint4 *) (x[t] + (int64_t) k * XS + 16);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t ok = 32 * (t0 + u * kRowWaves) + 8 * g < K ? 0xffffffffu : 0u;
+            const bf16x8_t wf = __builtin_bit_cast(bf16x8_t, make_uint4(wv[u].x & ok, wv[u].y & ok, wv[u].z & ok, wv[u].w & ok));
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                uint4 v = xv[u][t];
+                if constexpr (XF32) {
+                    const uint4 h = xw[u][t];
+                    v = make_uint4(pack_bf16x2(__uint_as_float(v.x), __uint_as_float(v.y)),
+                                   pack_bf16x2(__uint_as_float(v.z), __uint_as_float(v.w)),
+                                   pack_bf16x2(__uint_as_float(h.x), __uint_as_float(h.y)),
+                                   pack_bf16x2(__uint_as_float(h.z), __uint_as_float(h.w)));
+                }
+                v = make_uint4(v.x & ok, v.y & ok, v.z & ok, v.w & ok);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, v), wf, acc[t], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[wave][16 * t + 4 * g + r][r16] = acc[t][r];
+    __syncthreads();
+    for (int i = tid; i < 16 * NT * 16; i += kRowWaves * 64) {
+        const int64_t n = i >> 4, m = m0 + (i & 15);
+        if (n >= p.N || m >= p.M) continue;
+        float v = red[0][n][i & 15];
+#pragma unroll
+        for (int u = 1; u < kRowWaves; ++u) v += red[u][n][i & 15];
+        if (c.n) store_chain(p, c, n, m, v);
+        else store_out(p, p.y, p.res, n, m, v);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Host dispatch
 // ---------------------------------------------------------------------------
 static bool aligned16(const void * ptr) { return ((uintptr_t) ptr & 15) == 0; }
@@ -2292,6 +2407,45 @@ static void launch_gen_part(const GemmParams & p, bool wbf, bool xbf, float * pa
     }
 }
 
+// Whether gemm_row16 takes a product of at most 48 tokens with aligned rows: by
+// the bytes that a CU copies, its rounds of 16-feature workgroups times 32 K of
+// weights and each token tile's activations (f32 ones with their conversion
+// count 2.5 times, one token's a quarter: its lanes read the same bytes).  Both
+// launches of the K-split kernels against this one (us, bias epilogue, weights
+// from HBM; linear is a call of one product):
+//   row-major, 200 KB: 3072 x 1 x 3072 14.8 -> 9.5, 3072 x 8 x 3072 14.2 ->
+//   10.7, 1024 x 48 x 1024 12.2 -> 7.9, 4096 x 32 x 2048 14.1 -> 10.7; past it
+//   3072 x 32 x 3072 13.8 / 13.9 (295 KB), 9216 x 8 x 3072 21.0 / 23.1;
+//   tiled (whole 1 KB loads against kernels with less in flight), 600 KB: 3072 x
+//   1 x 3072 17.3 -> 8.1, 4096 x 48 x 2048 15.9 -> 11.8, 9216 x 1 x 3072 23.3 ->
+//   16.7, 3072 x 48 x 3072 16.4 -> 15.0 (393 KB); past it 9216 x 32 x 3072 21.6
+//   / 28.2.  gemm_skinny_wk keeps the wide ones it takes (14336 features).
+static bool skinny_wk_ok(const GemmParams & p, bool xf32);
+static bool row16_ok(const GemmParams & p, bool xf32, bool tiled) {
+    if (p.N > 48 || p.K % 8 != 0 || p.K < 32 || p.K > (1 << 24) || (tiled && skinny_wk_ok(p, xf32))) return false;
+    const double x = p.N == 1 ? 0.25 : (double) ((p.N + 15) / 16);
+    const double kb = std::ceil((double) p.M / 16 / 256) * (double) p.K * 32 / 1024 * (1 + x * (xf32 ? 2.5 : 1.0));
+    return kb <= (tiled ? 600 : 200);
+}
+
+static hipError_t run_row16(const GemmParams & p, bool xf32, bool tiled, const Chain & c, hipStream_t s) {
+    const dim3 grid((unsigned) ((p.M + 15) / 16)), block(kRowWaves * 64);
+#define WAMX_ROW16(NT)                                                                                    \
+    do {                                                                                                  \
+        if (xf32 && tiled) hipLaunchKernelGGL((gemm_row16<NT, true, true>), grid, block, 0, s, p, c);     \
+        else if (xf32) hipLaunchKernelGGL((gemm_row16<NT, true, false>), grid, block, 0, s, p, c);        \
+        else if (tiled) hipLaunchKernelGGL((gemm_row16<NT, false, true>), grid, block, 0, s, p, c);       \
+        else hipLaunchKernelGGL((gemm_row16<NT, false, false>), grid, block, 0, s, p, c);                 \
+    } while (0)
+    switch ((p.N + 15) / 16) {
+        case 1: WAMX_ROW16(1); break;
+        case 2: WAMX_ROW16(2); break;
+        default: WAMX_ROW16(3); break;
+    }
+#undef WAMX_ROW16
+    return hipGetLastError();
+}
+
 // f32 weights, or row-major bf16 weights with at most 64 tokens.
 static hipError_t run_gen(const GemmArgs & a, const GemmParams & p, hipStream_t s) {
     const bool wbf = a.w_type == WAMX_TYPE_BF16, xbf = a.x_type == WAMX_TYPE_BF16;
@@ -2488,6 +2642,7 @@ hipError_t launch_gemm_chain(const GemmArgs & a, const Chain & c, hipStream_t s)
     for (int k = 0; k < c.n; ++k)
         if (!aligned(c.st[k].a) || !aligned(c.st[k].out) || c.st[k].lda % 4 != 0 || !aligned16(c.st[k].gate))
             return hipErrorNotSupported;
+    if (wbf && vec_operands(a) && row16_ok(p, !xbf, false)) return run_row16(p, !xbf, false, c, s);
     const GenPlan b = gen_plan(p, wbf, xbf, 1, a.ws_bytes);
     if (b.splits <= 1) return hipErrorNotSupported;
     launch_gen_part(p, wbf, xbf, (float *) a.ws, b, 1, s);
@@ -2545,6 +2700,7 @@ hipError_t launch_gemm(const GemmArgs & a, hipStream_t s) {
     if (a.w_tiled && (!vec || batches != 1 || a.N > 64 || a.M % 16 != 0 || a.K % 32 != 0))
         return hipErrorNotSupported;
     if (a.w_tiled) {
+        if (row16_ok(p, xf32, true)) return run_row16(p, xf32, true, Chain{}, s);
         allow_skinny_lds();
         return run_skinny(p, xf32, a.ws, a.ws_bytes, s);
     }
@@ -2552,6 +2708,7 @@ hipError_t launch_gemm(const GemmArgs & a, hipStream_t s) {
     if (a.N <= 64) {
         const size_t need = vec && batches == 1 ? skinny_workspace_bytes(a.M, a.N, a.K) : 0;
         if (need && (!a.ws || need > a.ws_bytes || !aligned16(a.ws))) return hipErrorInvalidValue;
+        if (vec && batches == 1 && row16_ok(p, xf32, false)) return run_row16(p, xf32, false, Chain{}, s);
         return run_gen(a, p, s);
     }
     if (vec && !xf32 && batches == 1) {
