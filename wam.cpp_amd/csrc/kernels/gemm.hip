@@ -2652,26 +2652,51 @@ hipError_t launch_gemm_chain(const GemmArgs & a, const Chain & c, hipStream_t s)
     return hipGetLastError();
 }
 
+// V outputs per thread (4: M % 4 == 0 and 8-byte aligned rows).
+template <int V>
 __global__ __launch_bounds__(256) void partial_sum_bias(const float * __restrict__ part, int splits, int64_t N,
                                                         int64_t M, uint16_t * __restrict__ y,
                                                         uint16_t * __restrict__ out, int64_t ldy,
                                                         const uint16_t * __restrict__ bias) {
-    const int64_t total = N * M, i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+    typedef __attribute__((__vector_size__(V * sizeof(float)))) float fv_t;
+    const int64_t total = N * M, i = ((int64_t) blockIdx.x * 256 + threadIdx.x) * V;
     if (i >= total) return;
     const int64_t n = i / M, m = i % M;
-    float s = part[i];
-    for (int sp = 1; sp < splits; ++sp) s += part[sp * total + i];
-    const float v = round_bf16(s);
-    y[n * ldy + m] = f32_to_bf16(s);
-    out[n * ldy + m] = f32_to_bf16(v + bf16_to_f32(bias[n]));
+    const float b = bf16_to_f32(bias[n]);
+    fv_t s = *(const fv_t *) (part + i);
+    constexpr int kBatch = 8;
+    for (int sp0 = 1; sp0 < splits; sp0 += kBatch) {
+        fv_t v[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+            if (sp0 + u < splits) v[u] = *(const fv_t *) (part + (int64_t) (sp0 + u) * total + i);
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+            if (sp0 + u < splits) s += v[u];
+    }
+    if constexpr (V == 4) {
+        const uint2 h = make_uint2(pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]));
+        *(uint2 *) (y + n * ldy + m) = h;
+        *(uint2 *) (out + n * ldy + m) =
+            make_uint2(pack_bf16x2(round_bf16(s[0]) + b, round_bf16(s[1]) + b),
+                       pack_bf16x2(round_bf16(s[2]) + b, round_bf16(s[3]) + b));
+    } else {
+        y[n * ldy + m] = f32_to_bf16(s[0]);
+        out[n * ldy + m] = f32_to_bf16(round_bf16(s[0]) + b);
+    }
 }
 
 hipError_t launch_partial_sum(const float * part, int splits, int64_t N, int64_t M, void * y, int32_t y_type,
                               int64_t ldy, hipStream_t s, const void * bias, void * out) {
     if (out) {
         if (y_type != WAMX_TYPE_BF16) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(partial_sum_bias, dim3((unsigned) ((N * M + 255) / 256)), dim3(256), 0, s, part, splits, N,
-                           M, (uint16_t *) y, (uint16_t *) out, ldy, (const uint16_t *) bias);
+        const bool v4 = M % 4 == 0 && ldy % 4 == 0 && (((uintptr_t) y | (uintptr_t) out) & 7) == 0;
+        if (v4)
+            hipLaunchKernelGGL(partial_sum_bias<4>, dim3((unsigned) ((N * M / 4 + 255) / 256)), dim3(256), 0, s, part,
+                               splits, N, M, (uint16_t *) y, (uint16_t *) out, ldy, (const uint16_t *) bias);
+        else
+            hipLaunchKernelGGL(partial_sum_bias<1>, dim3((unsigned) ((N * M + 255) / 256)), dim3(256), 0, s, part,
+                               splits, N, M, (uint16_t *) y, (uint16_t *) out, ldy, (const uint16_t *) bias);
         return hipGetLastError();
     }
     GemmParams p{};

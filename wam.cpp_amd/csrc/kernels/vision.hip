@@ -130,9 +130,10 @@ __global__ __launch_bounds__(256) void conv_col_kernel(ConvDev c, int64_t b, int
 //
 // The column matrix this replaces was 9 times the image, written and read
 // back in workspace-sized pieces: 160 -> 160 channels, 3 x 3, 192 x 160 pixels
-// took 204 us of column kernels and 77 us of products in 3 pieces; now 9.6 us
-// of packing and 31 us of product (450 TFLOP/s; about 0.5 us per K step, of
-// which MFMAs and LDS reads account for 0.2).
+// took 204 us of column kernels, 77 us of products in 3 pieces and 31 us for the
+// bias; now 10 us of packing and 33 us of product that writes the convolution
+// and, with the bias node after it, its sum (425 TFLOP/s; about 0.5 us per K
+// step, of which MFMAs and LDS reads account for 0.2).
 // ---------------------------------------------------------------------------
 struct ConvGemm {
     const uint16_t * x;   // image b [IC][IH][IW]
@@ -234,13 +235,13 @@ __device__ __forceinline__ void conv_read(bf16x8_t (&fa)[FR], bf16x8_t (&fb)[2],
 // 32 FR output channels by 128 pixels per workgroup of 2 x 4 waves (16 FR
 // channels by 32 pixels each, MFMA 16x16x32; two waves per SIMD, so that one
 // reads its fragments while the other multiplies), K steps of 32 channels of
-// one tap through a ring of four LDS stages, three of them in flight.  Slot p
+// one tap, two between barriers, through a ring of six LDS stages.  Slot p
 // of a stage row holds 16-byte chunk p ^ ((row >> 2) & 3), which keeps the
 // fragment reads free of bank conflicts.  blockIdx.y: K slices, as f32
 // partials.
 template <int FR>
 __global__ __launch_bounds__(512) void conv_gemm_kernel(ConvGemm c) {
-    constexpr int BM = 32 * FR, BN = 128, ROWS = BM + BN, P = (ROWS + 127) / 128, E = ROWS * 32, S = 4;
+    constexpr int BM = 32 * FR, BN = 128, ROWS = BM + BN, P = (ROWS + 127) / 128, E = ROWS * 32, S = 6;
     __shared__ __align__(16) uint16_t st[S * E];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, r16 = lane & 15, wr = wave >> 2, wc = wave & 3;
@@ -300,25 +301,31 @@ __global__ __launch_bounds__(512) void conv_gemm_kernel(ConvGemm c) {
     const uint32_t slot = (r16 * 32 + (g ^ ((r16 >> 2) & 3)) * 8) * 2;
     const uint32_t base = (uint32_t) (uintptr_t) (const __attribute__((address_space(3))) void *) st + slot;
     const uint32_t aoff = 16 * FR * wr * 64, boff = (BM + 32 * wc) * 64;
-#pragma unroll
-    for (int i = 0; i < S - 1; ++i) dma();
-    uint32_t cur = base;
-    for (int kt = 0; kt < nk; ++kt) {
-        // The step's copies have landed once at most the next S - 2 stages' are
-        // outstanding; past the barrier the previous step's stage is free.
-        if (skip_last) __builtin_amdgcn_s_waitcnt(((S - 2) * (P - 1) & 0xF) | (7 << 4) | (0xF << 8));
-        else __builtin_amdgcn_s_waitcnt(((S - 2) * P & 0xF) | (7 << 4) | (0xF << 8));
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        dma();
+    auto step = [&](uint32_t at) {
         bf16x8_t a[FR], b[2];
-        conv_read<FR>(a, b, cur + aoff, cur + boff);
-        cur = cur == base + (S - 1) * E * 2 ? base : cur + E * 2;
+        conv_read<FR>(a, b, at + aoff, at + boff);
 #pragma unroll
         for (int i = 0; i < FR; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    };
+#pragma unroll
+    for (int i = 0; i < S - 2; ++i) dma();
+    uint32_t cur = base;
+    for (int kt = 0; kt < nk; kt += 2) {
+        // Two steps per barrier.  Their copies have landed once at most the next
+        // two steps' are outstanding; past the barrier the previous two stages
+        // are free.
+        if (skip_last) __builtin_amdgcn_s_waitcnt((2 * (P - 1) & 0xF) | (7 << 4) | (0xF << 8));
+        else __builtin_amdgcn_s_waitcnt((2 * P & 0xF) | (7 << 4) | (0xF << 8));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        dma();
+        dma();
+        step(cur);
+        if (kt + 1 < nk) step(cur + E * 2);
+        cur = cur == base + (S - 2) * E * 2 ? base : cur + 2 * E * 2;
     }
     __builtin_amdgcn_s_waitcnt((7 << 4) | (0xF << 8));  // the trailing copies land before the workgroup's LDS is reused
 
@@ -381,12 +388,13 @@ static hipError_t conv_implicit(const ConvDev & d, const void * kernel, void * d
             const int image = (int) ((IWp + kPackPix - 1) / kPackPix * (ICp / 32) * c.rows);
             const int kblocks = b == 0 && oy == 0 ? (int) ((OC * taps * (ICp / 8) + 255) / 256) : 0;
             hipLaunchKernelGGL(conv_pack_kernel, dim3((unsigned) (image + kblocks)), dim3(256), 0, s, c, image);
-            // K slices up to about two workgroups (of the LDS ring's size) per CU, of 6 steps or more.
+            // K slices up to one workgroup per CU (the ring allows no second), of
+            // 8 steps or more.  640 -> 640 channels, 3 x 3, 48 x 40 pixels in 4
+            // slices 53.8 us with packing and bias, in 8 63.8.
             const int64_t tiles = (OC + 32 * fr - 1) / (32 * fr) * ((c.pix + 127) / 128);
             const size_t room = (size_t) ((char *) c.xp - (char *) ws);
-            int64_t splits = std::max<int64_t>(1, std::min<int64_t>(512 / tiles, ktot / 6));
+            int64_t splits = std::max<int64_t>(1, std::min<int64_t>(256 / tiles, ktot / 8));
             splits = std::min<int64_t>(splits, (int64_t) (room / ((size_t) OC * c.pix * 4)));
-            if (tiles > 170) splits = 1;
             splits = std::max<int64_t>(splits, 1);
             c.ksteps = (int) ((ktot + splits - 1) / splits);
             splits = (ktot + c.ksteps - 1) / c.ksteps;
