@@ -97,6 +97,7 @@ def test_modulo_broadcast(wx, be, rng, bs):
 
 
 @pytest.mark.parametrize("dim,sa,sb", [
+    (0, (2, 3, 5, 1), (2, 3, 5, 511)), (0, (1, 2, 7, 1000), (1, 2, 7, 1)), (0, (1, 3, 2, 2043), (1, 3, 2, 13)),
     (0, (2, 3, 5, 1), (2, 3, 5, 48)), (0, (1, 24, 128, 49), (1, 24, 128, 3072)), (0, (1, 2, 3, 8), (1, 2, 3, 16)),
     (1, (1, 24, 1, 128), (1, 24, 48, 128)), (1, (1, 24, 49, 128), (1, 24, 3072, 128)), (2, (2, 3, 5, 7), (2, 4, 5, 7)),
     (3, (1, 3, 4, 8), (2, 3, 4, 8))])

@@ -81,8 +81,8 @@ __global__ void copy_kernel(Ref4 src, Ref4 dst, int64_t n) {
 // divisions per operand and element and on 2- or 4-byte accesses; here the
 // index takes at most three multiplications for 8 elements.  Measured: ADD of
 // a [192, 160, 160] bf16 image and a per-channel bias 31 -> 7.6 us, concatenation
-// of 9.6 M bf16 along dim 1 42 -> 9.5 us, along dim 0 at odd offsets (one
-// element per thread) 42 -> 26 us.
+// of 9.6 M bf16 along dim 1 42 -> 9.5 us (along dim 0 at odd offsets:
+// concat0_kernel).
 // ---------------------------------------------------------------------------
 // n / d for n < 2^31 by a multiplication (Granlund and Montgomery, "Division by
 // Invariant Integers using Multiplication", 1994, figure 4.1: m' = floor(2^32
@@ -226,6 +226,29 @@ __global__ __launch_bounds__(256) void map_kernel(MapArgs m) {
             for (int e = 0; e < V; ++e) x[e] = OP == kMapAdd ? x[e] + y[e] : x[e] * y[e];
         }
         map_store<V>(m.d.type, d, x);
+    }
+}
+
+// Concatenation along dim 0 of 2-byte elements at any offset (a cache's V^T
+// rows behind a state token's: odd row lengths), 8 per thread at the element's
+// own alignment, which gfx950's global accesses take; the chunk that holds the
+// seam or the row's end goes element by element.  One workgroup row per row.
+struct __attribute__((packed, aligned(2))) loose16_t {
+    uint32_t x, y, z, w;
+};
+__global__ __launch_bounds__(256) void concat0_kernel(Ref4 a, Ref4 b, Ref4 dst) {
+    const int64_t row = blockIdx.y, i1 = row % dst.ne1, i2 = row / dst.ne1 % dst.ne2, i3 = row / (dst.ne1 * dst.ne2);
+    const int64_t i0 = 8 * ((int64_t) blockIdx.x * 256 + threadIdx.x);
+    if (i0 >= dst.ne0) return;
+    const uint16_t * pa = (const uint16_t *) at(a, 0, i1, i2, i3);
+    const uint16_t * pb = (const uint16_t *) at(b, 0, i1, i2, i3) - a.ne0;
+    uint16_t * pd = (uint16_t *) at(dst, 0, i1, i2, i3);
+    if (i0 + 8 <= a.ne0) {
+        *(loose16_t *) (pd + i0) = *(const loose16_t *) (pa + i0);
+    } else if (i0 >= a.ne0 && i0 + 8 <= dst.ne0) {
+        *(loose16_t *) (pd + i0) = *(const loose16_t *) (pb + i0);
+    } else {
+        for (int64_t i = i0; i < min(i0 + 8, dst.ne0); ++i) pd[i] = i < a.ne0 ? pa[i] : pb[i];
     }
 }
 
@@ -848,6 +871,14 @@ hipError_t launch_unary(int op, const TensorRef & a, const TensorRef & dst, floa
 hipError_t launch_concat(const TensorRef & a, const TensorRef & b, const TensorRef & dst, int dim, hipStream_t s) {
     const int64_t n = nel(dst);
     if (n <= 0) return hipSuccess;
+    const int64_t rows = dst.ne[1] * dst.ne[2] * dst.ne[3];
+    if (dim == 0 && dst.type != WAMX_TYPE_F32 && dst.type != WAMX_TYPE_I32 && a.nb[0] == 2 && b.nb[0] == 2 &&
+        dst.nb[0] == 2 && dst.ne[0] >= 512 && rows <= 65535 && (a.ne[0] % 8 || dst.ne[0] % 8)) {
+        // 9.6 M elements in rows of 3121: 26 us one element per thread, 15.3 so.
+        hipLaunchKernelGGL(concat0_kernel, dim3((unsigned) ((dst.ne[0] + 2047) / 2048), (unsigned) rows), dim3(256), 0,
+                           s, to_ref4(a), to_ref4(b), to_ref4(dst));
+        return hipGetLastError();
+    }
     if (try_map<kMapConcat>(a, &b, dst, 0, 0, 0, dim, s)) return hipGetLastError();
     hipLaunchKernelGGL(concat_kernel, grid1d(n), dim3(256), 0, s, to_ref4(a), to_ref4(b), to_ref4(dst), dim, n);
     return hipGetLastError();
