@@ -2652,11 +2652,11 @@ hipError_t launch_gemm_chain(const GemmArgs & a, const Chain & c, hipStream_t s)
     return hipGetLastError();
 }
 
-// V outputs per thread (4: M % 4 == 0 and 8-byte aligned rows).
+// V outputs per thread (4: M % 4 == 0 and 8-byte aligned rows).  y and out may
+// be the same array (the sum in place).
 template <int V>
 __global__ __launch_bounds__(256) void partial_sum_bias(const float * __restrict__ part, int splits, int64_t N,
-                                                        int64_t M, uint16_t * __restrict__ y,
-                                                        uint16_t * __restrict__ out, int64_t ldy,
+                                                        int64_t M, uint16_t * y, uint16_t * out, int64_t ldy,
                                                         const uint16_t * __restrict__ bias) {
     typedef __attribute__((__vector_size__(V * sizeof(float)))) float fv_t;
     const int64_t total = N * M, i = ((int64_t) blockIdx.x * 256 + threadIdx.x) * V;
