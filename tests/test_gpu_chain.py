@@ -131,3 +131,55 @@ def test_conv_bias_same_bits_as_nodes_apart(wx, be, IC, OC, IW, IH, B):
     finally:
         g.close()
     assert np.array_equal(out, apart)
+
+
+@pytest.mark.parametrize("node,IC,OC,IW,IH", [(n, *s) for n in ("gelu", "bias_gelu") for s in
+                                              ((32, 160, 40, 33), (640, 640, 12, 10), (32, 1, 40, 33))] +
+                         [("gated", 32, 1, 40, 33)])  # 2-D tensors only
+def test_conv_before_other_nodes_runs_apart(wx, be, node, IC, OC, IW, IH):
+    """A convolution followed by GELU, bias + GELU (a bias per column of the
+    image: more output channels than bias values) or, with one output channel,
+    a gated residual: nodes that its epilogue does not know, in one K slice and
+    in several.  The same bits as the node on the fetched convolution."""
+    print(f"conv + {node} {IC}->{OC} {IW}x{IH}", flush=True)
+    rng = np.random.default_rng(IC + OC)
+    lib = be.lib
+    k, x, row, full = (wx.f32_to_bf16(rng.standard_normal(s).astype(np.float32))
+                       for s in ((OC, IC, 3, 3), (1, IC, IH, IW), (IW,), (IH, IW)))
+    gate = rng.standard_normal(IW).astype(np.float32)
+
+    def run(conv):
+        """(convolution, node): the node after the convolution, or on `conv`."""
+        g = Graph(wx, be)
+        try:
+            sets, outs = [], []
+            def leaf(a, typ, *ne):
+                t = g.t(typ, *ne)
+                sets.append((t, a))
+                return t
+            if conv is None:
+                cur = lib.wamx_conv_2d_direct(g.ctx, leaf(k, wx.TYPE_BF16, 3, 3, IC, OC),
+                                              leaf(x, wx.TYPE_BF16, IW, IH, IC, 1), 1, 1, 1, 1, 1, 1)
+                outs.append(cur)
+            else:
+                cur = leaf(conv, wx.TYPE_BF16, IW, IH, OC, 1)
+            if node == "gelu":
+                y = lib.wamx_gelu(g.ctx, cur)
+            elif node == "bias_gelu":
+                y = lib.wamx_bias_gelu_bf16(g.ctx, cur, leaf(row, wx.TYPE_BF16, IW))
+            else:
+                y = lib.wamx_gated_residual_bf16(g.ctx, leaf(full, wx.TYPE_BF16, IW, IH), cur,
+                                                 leaf(gate, wx.TYPE_F32, IW))
+            assert y, wx.last_error()
+            outs.append(y)
+            g.alloc()
+            for t, a in sets:
+                g.set(t, a)
+            g.compute(y)
+            return [g.get(t, np.uint16, (1, OC, IH, IW)) for t in outs]
+        finally:
+            g.close()
+
+    conv, got = run(None)
+    apart, = run(conv)
+    assert np.array_equal(got, apart)

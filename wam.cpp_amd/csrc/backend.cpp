@@ -594,6 +594,8 @@ static int match_chain(wamx_cgraph * g, int i, int n, bool lanes, bool placed, C
     for (int j = next_compute(g, i, n, lanes); j < n && c.n < (conv ? 1 : kMaxStages); j = next_compute(g, j, n, lanes)) {
         const wamx_tensor * t = wamx_graph_node(g, j);
         if (t->type != typ || !wamx_are_same_shape(t, prod) || !wamx_is_contiguous(t) || (placed && !t->data)) break;
+        // A convolution's launches add a bias and nothing else.
+        if (conv && (t->op != WAMX_OP_ADD || t->src[2])) break;
         ChainStage st;
         const wamx_tensor * o = nullptr;     // the operand
         const wamx_tensor * gate = nullptr;
@@ -665,9 +667,11 @@ static int match_chain(wamx_cgraph * g, int i, int n, bool lanes, bool placed, C
 }
 
 static hipError_t run_chain(wamx_backend * be, const wamx_tensor * node, const Chain & c) {
-    if (node->op == WAMX_OP_CONV_2D)
+    if (node->op == WAMX_OP_CONV_2D) {
+        if (c.n != 1 || c.st[0].kind != kStageAddRow) return hipErrorNotSupported;
         return launch_conv2d(ref_of(node->src[0]), ref_of(node->src[1]), ref_of(node), node->op_params, be->cws,
                              kWorkspaceBytes, be->cs, c.st[0].a, c.st[0].out);
+    }
     return launch_gemm_chain(mul_mat_args(be, node), c, be->cs);
 }
 
