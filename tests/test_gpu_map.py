@@ -132,3 +132,27 @@ def test_soft_max_rows(wx, be, rng, n, mask):
         assert np.allclose(got, e / e.sum(-1, keepdims=True), rtol=32 * 2.0 ** -24, atol=0)
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("mask", [False, True])
+def test_soft_max_rows_of_no_elements(wx, be, rng, mask):
+    """Nothing to read or write: the graph runs, and the soft_max of the
+    tensor beside it in memory is what it is without the empty one."""
+    print(f"soft_max rows of 0 mask={mask}", flush=True)
+    x = rng.standard_normal((1, 1, 5, 7)).astype(np.float32)
+    got = []
+    for empty in (False, True):
+        g = G(wx, be)
+        try:
+            outs = [be.lib.wamx_soft_max_ext(g.ctx, g.leaf(wx, x, "f32"), None, 1.0, 0.0)]
+            if empty:
+                m = g.t(wx.TYPE_F32, 0, 5) if mask else None
+                outs.insert(0, be.lib.wamx_soft_max_ext(g.ctx, g.t(wx.TYPE_F32, 0, 5), m, 0.125, 0.0))
+                assert outs[0], wx.last_error()
+            g.alloc()
+            g.set(*g.todo[0])
+            g.compute(*outs)
+            got.append(g.get(outs[-1], np.float32, x.shape))
+        finally:
+            g.close()
+    assert np.array_equal(*got)

@@ -894,7 +894,7 @@ hipError_t launch_get_rows(const TensorRef & a, const int32_t * rows, const Tens
 hipError_t launch_softmax_f32(const TensorRef & x, const TensorRef & mask, const TensorRef & y, float scale,
                               hipStream_t s) {
     const int64_t rows = x.ne[1] * x.ne[2] * x.ne[3];
-    if (rows <= 0) return hipSuccess;
+    if (rows <= 0 || x.ne[0] <= 0) return hipSuccess;  // the kernel loads a row's last element for lanes past it
 #define WAMX_SOFTMAX(PER, W)                                                                                       \
     hipLaunchKernelGGL((softmax_kernel<PER, W>), dim3((unsigned) rows), dim3(64 * W), 0, s, to_ref4(x), to_ref4(mask), \
                        to_ref4(y), scale)
