@@ -26,6 +26,7 @@ import pytest
 import ggml_mirror as gm
 from conftest import assert_parity
 from test_gpu_dropin import Runner
+from test_gpu_fusion import Graph
 
 pytestmark = pytest.mark.gpu
 
@@ -151,3 +152,24 @@ def test_bf16_conv_integers_exact(wx, be, orc, IC, OC, KW, KH, s, p, d, IW, IH, 
     ref = orc.conv_2d(k, x, s[0], s[1], p[0], p[1], d[0], d[1])
     assert ref.shape == (B, OC, y.ne[1], y.ne[0])
     assert np.array_equal(r.fetch(y, np.uint16, ref.shape), _bf(wx, ref))
+
+
+@pytest.mark.parametrize("typ", ["bf16", "f32"])
+@pytest.mark.parametrize("IC,OC,B,ok", [(32, 0, 1, True), (32, 8, 0, True), (0, 8, 1, False)])
+def test_conv_with_an_empty_extent(wx, be, typ, IC, OC, B, ok):
+    """No output channels or no images: nothing to compute, the graph runs.
+    No input channels: refused with an error."""
+    print(f"conv {IC}->{OC} x{B} {typ}", flush=True)
+    T = wx.TYPE_BF16 if typ == "bf16" else wx.TYPE_F32
+    g = Graph(wx, be)
+    try:
+        y = be.lib.wamx_conv_2d_direct(g.ctx, g.t(T, 3, 3, IC, OC), g.t(T, 9, 8, IC, B), 1, 1, 1, 1, 1, 1)
+        assert y, wx.last_error()
+        g.alloc()
+        if ok:
+            g.compute(y)
+        else:
+            with pytest.raises(RuntimeError):
+                g.compute(y)
+    finally:
+        g.close()

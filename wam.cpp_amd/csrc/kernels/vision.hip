@@ -440,6 +440,8 @@ hipError_t launch_conv2d(const TensorRef & kernel, const TensorRef & input, cons
     c.d1 = pp[5];
     const int64_t K = c.IC * c.KH * c.KW, P = c.OW * c.OH, OC = kernel.ne[3], B = input.ne[3];
     const size_t es = bf ? 2 : 4;
+    if (OC <= 0 || B <= 0 || P <= 0) return hipSuccess;  // no output
+    if (K <= 0) return hipErrorInvalidValue;
     if (bf) {
         const hipError_t e = conv_implicit(c, kernel.data, dst.data, bias, out, OC, B, ws, ws_bytes, s);
         if (e != hipErrorNotSupported) return e;
