@@ -156,3 +156,29 @@ def test_soft_max_rows_of_no_elements(wx, be, rng, mask):
         finally:
             g.close()
     assert np.array_equal(*got)
+
+
+@pytest.mark.parametrize("n", [1, 7, 520, 70001])
+@pytest.mark.parametrize("src,dst", [("f32", "f32"), ("f32", "bf16"), ("bf16", "f32")])
+@pytest.mark.parametrize("side", ["src", "dst"])
+def test_reshaping_copy_of_a_transposed_row(wx, be, rng, n, src, dst, side):
+    """A row [n] seen as [1, n] through a transpose: dense, but the stride of
+    its first dim (one element) is the whole row.  Copied to, or filled from,
+    a tensor of another shape, in memory order."""
+    print(f"reshaping copy {n} {src}->{dst} transposed {side}", flush=True)
+    a = rng.standard_normal((1, 1, 1, n)).astype(np.float32)
+    g = G(wx, be)
+    try:
+        x = g.leaf(wx, a, src)
+        d = g.t(TYPES[dst], n)
+        if side == "src":
+            y = be.lib.wamx_cpy(g.ctx, be.lib.wamx_transpose(g.ctx, x), d)
+        else:
+            y = be.lib.wamx_cpy(g.ctx, x, be.lib.wamx_transpose(g.ctx, d))
+        assert y, wx.last_error()
+        g.alloc()
+        g.set(*g.todo[0])
+        g.compute(y)
+        assert np.array_equal(g.get(d, {"f32": np.float32, "bf16": np.uint16}[dst], a.shape), to_bits(wx, value(wx, a, src), dst))
+    finally:
+        g.close()

@@ -840,6 +840,7 @@ hipError_t launch_copy(const TensorRef & src, const TensorRef & dst, hipStream_t
     if (!same_shape && dense(src) && dense(dst)) {  // a reshape: both in memory order
         TensorRef f = src, d = dst;
         for (TensorRef * t : {&f, &d}) {
+            t->nb[0] = type_bytes(t->type);  // a first dim of one element may have any stride
             t->ne[0] = n;
             t->ne[1] = t->ne[2] = t->ne[3] = 1;
         }
