@@ -2,12 +2,14 @@
 row ops that consume its output (LayerNorm / adaLN modulation of the residual
 stream; RMSNorm + RoPE of the Q and K column ranges and the V^T copy) runs as
 the skinny GEMM plus one reduce that applies the row ops; on eight 48-token
-chunks (384 rows, the batched denoise step) as the K-sliced 128 x 128 GEMM
+chunks (384 rows, the batched denoise step) as the K-sliced tiled GEMM
 plus the same reduce, with chunk-major Q/K and V^T destinations.  The fused graph
 must produce the same bits as the standalone ops launched one at a time
 (wamx_op_linear, wamx_op_norm_modulation_bf16 / wamx_op_layer_norm_bf16,
 wamx_op_qk_norm_rope and a host transpose for V^T), which the per-op tests
-hold to the oracle.
+hold to the oracle.  Products of 2 to 48 tokens that run in one launch when
+alone sum in another f32 order there: the row op is the same bits on the fused
+product, and the two products differ by no more than the order of the sum.
 """
 from __future__ import annotations
 
@@ -168,6 +170,83 @@ def test_qkv_split_is_bit_exact(wx, be, rng, T):
         assert np.array_equal(got_vt, rq[:, 2 * D:].reshape(T, H, DH).transpose(1, 2, 0))
     finally:
         g.close()
+
+
+def _linear_norm(wx, be, rng, M, K, T, tiled, epi):
+    """LINEAR -> LayerNorm in one graph, and the same LINEAR alone through
+    wamx_op_linear[_tiled]: (w, x, fused product, fused norm, product alone,
+    norm of the product alone, norm of the fused product)."""
+    lib = be.lib
+    g, tctx, tbuf = Graph(wx, be), lib.wamx_init(4), None
+    try:
+        w = lib.wamx_new_tensor_2d(tctx if tiled else g.ctx, wx.TYPE_BF16, K, M)
+        x, h = g.t(wx.TYPE_BF16, K, T), g.t(wx.TYPE_BF16, M, T)
+        b, sc, sh, gate = g.t(wx.TYPE_BF16, M), g.t(wx.TYPE_BF16, M), g.t(wx.TYPE_BF16, M), g.t(wx.TYPE_F32, M)
+        gated = epi == wx.EPI_BIAS_GATED
+        y = lib.wamx_linear(g.ctx, w, x, b if gated else None, epi, h if gated else None, gate if gated else None)
+        n = lib.wamx_layer_norm_bf16(g.ctx, y, sc, sh, 1e-6)
+        if tiled:
+            tbuf = lib.wamx_backend_alloc_ctx_tensors_from_buft(tctx, lib.wamx_backend_tiled_buffer_type(0))
+            assert tbuf and w.contents.extra, wx.last_error()
+        g.alloc()
+        bf = lambda a: wx.f32_to_bf16(np.asarray(a, np.float32))  # noqa: E731
+        hw, hx = bf(rng.standard_normal((M, K)) * 0.02), bf(rng.standard_normal((T, K)))
+        for t, a in ((w, hw), (x, hx), (h, bf(rng.standard_normal((T, M)))), (b, bf(rng.standard_normal(M) * 0.02)),
+                     (sc, bf(1 + 0.1 * rng.standard_normal(M))), (sh, bf(0.1 * rng.standard_normal(M))),
+                     (gate, (0.5 * rng.standard_normal(M)).astype(np.float32))):
+            g.set(t, a)
+        g.compute(n)
+        got = [g.get(t, np.uint16, (T, M)) for t in (y, n)]
+        alone, norm = be.empty(T * M * 2), be.empty(T * M * 2)
+        op = lib.wamx_op_linear_tiled if tiled else lib.wamx_op_linear
+        wx.check(op(be.ptr, data(w), data(x), wx.TYPE_BF16, data(b) if gated else None, epi,
+                    data(h) if gated else None, C.cast(data(gate), C.POINTER(C.c_float)) if gated else None,
+                    alone.ptr, M, T, K))
+        out = [alone.download(np.uint16, (T, M))]
+        for ptr in (alone.ptr, data(y)):
+            wx.check(lib.wamx_op_layer_norm_bf16(be.ptr, ptr, M, data(sc), data(sh), norm.ptr, T, M, 1e-6))
+            be.sync()
+            out.append(norm.download(np.uint16, (T, M)))
+        return [hw, hx] + got + out
+    finally:
+        g.close()
+        if tbuf:
+            lib.wamx_buffer_free(tbuf)
+        lib.wamx_free(tctx)
+
+
+# One token in one launch per product (tiled and row-major), and the tiles and
+# K slices of each kind above 64 tokens (3072 x 14336: 16 slices of 192 x 192
+# at 192 tokens, 8 of them at 384, 8 of 256 x 256 at 512; 16 of 128 x 128 at 65).
+@pytest.mark.parametrize("M,K,T,tiled", [(3072, 3072, 1, True), (3072, 14336, 1, True), (1024, 1024, 1, False),
+                                         (3072, 14336, 65, False), (3072, 14336, 192, False),
+                                         (3072, 14336, 384, False), (3072, 14336, 512, False)])
+def test_linear_then_norm_sums_as_the_product_alone(wx, be, rng, M, K, T, tiled):
+    print(f"fusion linear->norm {M}x{T}x{K} tiled={tiled}", flush=True)
+    _, _, y, n, alone, norm_alone, _ = _linear_norm(wx, be, rng, M, K, T, tiled, wx.EPI_BIAS_GATED)
+    assert np.array_equal(y, alone)
+    assert np.array_equal(n, norm_alone)
+
+
+@pytest.mark.parametrize("T", [192, 512])
+def test_qkv_split_many_tokens_is_bit_exact(wx, be, rng, T):
+    """9216 x 3072 in 4 slices of 192 x 192 tiles and 3 of 256 x 256."""
+    test_qkv_split_is_bit_exact(wx, be, rng, T)
+
+
+@pytest.mark.parametrize("M,K,T,tiled", [(3072, 3072, 48, True), (2048, 2048, 20, True), (3072, 3072, 8, False),
+                                         (1024, 1024, 48, False)])
+def test_few_token_products_sum_in_another_order_alone(wx, be, rng, M, K, T, tiled):
+    """Products of 2 to 48 tokens that take one launch when alone: both sums
+    are within K f32 roundings (2^-23, a truncating adder's) of the exact one
+    and rounded to bf16 once (2^-8); the norm is that of the fused product."""
+    print(f"fusion few tokens {M}x{T}x{K} tiled={tiled}", flush=True)
+    w, x, y, n, alone, _, norm_fused = _linear_norm(wx, be, rng, M, K, T, tiled, wx.EPI_NONE)
+    assert np.array_equal(n, norm_fused)
+    fw, fx = (np.abs(wx.bf16_to_f32(a)).astype(np.float64) for a in (w, x))
+    a, b = (wx.bf16_to_f32(v).astype(np.float64) for v in (y, alone))
+    assert np.all(np.abs(a - b) <= 2 * K * 2.0 ** -23 * (fx @ fw.T) + 2 * 2.0 ** -8 * np.maximum(np.abs(a), np.abs(b)))
+    assert np.mean(y != alone) < 0.02  # most sums round alike
 
 
 def test_qkv_row_ops_apart_are_not_fused(wx, be, rng):

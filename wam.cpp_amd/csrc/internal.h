@@ -61,9 +61,10 @@ hipError_t tensor_set_from_device(wamx_tensor * t, const void * src, hipStream_t
 size_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K);
 // Workspace of a backend: K-split GEMM and key-split attention partials.
 constexpr size_t kBackendWorkspaceBytes = 64ull << 20;
-// Bytes of fp32 K-split partials that launch_gemm writes to its workspace
-// for a plain bf16-weight product (row-major, contiguous, one batch) of N
-// tokens, given ws_bytes of workspace; 0 when the product takes no K split.
+// Bytes of fp32 K-split partials by which wamx_op_linear_noalloc refuses a
+// bf16-weight product (row-major, contiguous, one batch) of N tokens, given
+// ws_bytes of workspace: an upper limit kept from earlier plans, not what
+// launch_gemm writes (never more than the workspace).
 size_t linear_split_bytes(int64_t M, int64_t N, int64_t K, int32_t x_type, size_t ws_bytes);
 
 // y[n][m] (row stride ldy) = sum over splits of part[split][n][m], in split
@@ -114,10 +115,10 @@ struct RowPost {
     int64_t width = 0, head_dim = 0;
     RowSeg seg[3];
 };
-// The split-K GEMM whose reduce applies `post`: the skinny part kernel for up
-// to 64 tokens, the K-sliced 128 x 128 DMA GEMM for more tokens on grids
-// that it splits (the batched denoise step).  Returns hipErrorNotSupported,
-// launching nothing, when the product or the row op does not fit that path.
+// The product as f32 planes and a reduce that applies `post`: the few-token
+// kernels for up to 64 tokens, the K slices that launch_gemm takes for more
+// (the batched denoise step).  Returns hipErrorNotSupported, launching nothing,
+// when the product or the row op does not fit that path.
 hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStream_t s);
 
 // Element-wise nodes that follow a product, applied by its last launch: v is the product's value as its node stores it, each stage's result

@@ -549,7 +549,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void gemm_dma(GemmParams p, int 
     __shared__ __align__(16) uint16_t st1[E];
     __shared__ __align__(16) uint16_t st2[S > 2 ? E : 8];
     __shared__ __align__(16) uint16_t st3[S > 3 ? E : 8];
-    // Batches along blockIdx.y (run_dma_splitk: K slices, each into its own
+    // Batches along blockIdx.y (launch_dma_splitk_parts: K slices, each into its own
     // f32 partial plane): x, w and y advance by their batch strides.
     if (blockIdx.y) {
         const int64_t z = blockIdx.y;
@@ -789,7 +789,7 @@ __global__ __launch_bounds__(64 * WM * WN * (SCHED == kSchedProducer ? 2 : 1), 1
         if (i * RPI < BM) soff[i] = (uint32_t) ((min(n0 + r, N - 1) * p.ldx + 8 * c) * 2);
         else soff[i] = (uint32_t) ((min(m0 + min(r - BM, BN - 1), M - 1) * p.ldw + 8 * c) * 2);
     }
-    // K slices along blockIdx.y (launch_pipe_splitk): p.K columns each, into
+    // K slices along blockIdx.y (launch_pipe_parts): p.K columns each, into
     // f32 partial planes.
     const int64_t slice = blockIdx.y;
     const char * const xb = (const char *) p.x + slice * p.K * 2, * const wb = (const char *) p.w + slice * p.K * 2;
@@ -1279,9 +1279,11 @@ __global__ __launch_bounds__(256) void gemm_reduce_chain(GemmParams p, Chain c, 
 // launches (part + this) instead of three.  One workgroup per token (and
 // segment); thread c owns 8-column chunk c, which is the chunk layout of the
 // standalone row kernels (norm_mod_bf16_vec / qk_norm_rope_vec with one chunk
-// per thread), and the row arithmetic is shared with them (rowops.h), so the
-// fused and unfused paths give the same bits.  The GEMM output row is written
-// as well (16-byte chunks).
+// per thread), and the row arithmetic is shared with them (rowops.h), so they
+// give the same bits on the same product.  The product's own sums are those of
+// launch_gemm but for its two few-token kernels that split K inside a workgroup
+// (see launch_gemm_rowpost).  The GEMM output row is written as well (16-byte
+// chunks).
 //   POST kPostNormAffine / kPostNormModF32 / kPostNormModBf16: LayerNorm of
 //     the row (weights, or adaLN modulation in f32 / bf16) into rp.out;
 //   POST kPostSegs: up to three segments of rp.width columns, one per
@@ -1560,10 +1562,10 @@ size_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 static int64_t tiles_of(const GemmParams & p, int bm, int bn);
 static int dma_splitk_plan(const GemmParams & p, size_t ws_bytes);
 
-// The K split of a plain product with row-major weights: the few-token limit
-// up to 64 tokens, else the K-sliced 128 x 128 GEMM that
-// dispatch_dma runs for bf16 activations on grids too small for the 256 /
-// 192 tiles (whose slice count depends on the workspace size).
+// The partials by which wamx_op_linear_noalloc has always refused a product
+// with row-major weights: the few-token limit up to 64 tokens, else those of
+// 128 x 128 tiles on grids too small for whole 256 / 192 tiles.  What launch_gemm
+// writes is its own plans' (gen_plan, dma_plan), never more than the workspace.
 size_t linear_split_bytes(int64_t M, int64_t N, int64_t K, int32_t x_type, size_t ws_bytes) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     if (N <= 64) return skinny_workspace_bytes(M, N, K);
@@ -2104,23 +2106,28 @@ static hipError_t run_dma_pipe(const GemmParams & p, hipStream_t s) {
     return launch_dma_pipe<BM, BN, WM, WN, S, SCHED, BKP>(p, s);
 }
 
-// K slices of the pipelined kernel into f32 partial planes of ws, each of
-// p.K / splits columns, then the reduce with the epilogue.
-template <int BM, int BN, int WM, int WN, int S, int SCHED, int BKP>
-static hipError_t launch_pipe_splitk(const GemmParams & p, int splits, void * ws, hipStream_t s) {
+// The product's parameters with f32 partial planes [N][M] at ws as its output
+// and no epilogue.
+static GemmParams plane_params(const GemmParams & p, void * ws) {
     GemmParams q = p;
-    q.K = p.K / splits;
     q.y = ws;
     q.y_type = WAMX_TYPE_F32;
     q.ldy = p.M;
     q.epi = WAMX_EPI_NONE;
     q.vec_out = 0;
+    return q;
+}
+
+// K slices of the pipelined kernel into partial planes of ws, each of
+// p.K / splits columns.
+template <int BM, int BN, int WM, int WN, int S, int SCHED, int BKP>
+static void launch_pipe_parts(const GemmParams & p, int splits, void * ws, hipStream_t s) {
+    GemmParams q = plane_params(p, ws);
+    q.K = p.K / splits;
     const int nt_m = (int) ((p.M + BN - 1) / BN), nt_n = (int) ((p.N + BM - 1) / BM);
     const int threads = 64 * WM * WN * (SCHED == kSchedProducer ? 2 : 1);
     hipLaunchKernelGGL((gemm_dma_pipe<BM, BN, WM, WN, S, SCHED, BKP>), dim3((unsigned) (nt_m * nt_n), (unsigned) splits),
                        dim3(threads), 0, s, q, nt_m, nt_n);
-    launch_reduce(p, (const float *) ws, splits, s);
-    return hipGetLastError();
 }
 
 static int64_t tiles_of(const GemmParams & p, int bm, int bn) { return ((p.N + bm - 1) / bm) * ((p.M + bn - 1) / bn); }
@@ -2169,29 +2176,18 @@ static int dma_splitk_plan(const GemmParams & p, size_t ws_bytes) {
 }
 
 // K split over blockIdx.y of gemm_dma<128, 128>: slice z multiplies K columns
-// [z*K/s, (z+1)*K/s) into f32 partial plane z of ws, then gemm_skinny_reduce
-// sums the planes in slice order (deterministic) and applies the epilogue.
+// [z*K/s, (z+1)*K/s) into f32 partial plane z of ws.
 static void launch_dma_splitk_parts(const GemmParams & p, int splits, void * ws, hipStream_t s) {
-    GemmParams q = p;
+    GemmParams q = plane_params(p, ws);
     const int64_t ks = p.K / splits;
     q.K = ks;
     q.x_bs2 = ks;
     q.w_bs2 = ks;
-    q.y = ws;
-    q.y_type = WAMX_TYPE_F32;
-    q.ldy = p.M;
     q.y_bs2 = p.N * p.M;
-    q.epi = WAMX_EPI_NONE;
-    q.vec_out = 0;
     const int nt_m = (int) ((p.M + 127) / 128), nt_n = (int) ((p.N + 127) / 128);
     constexpr int occ = dma_occupancy<128, 128, 2, 2, 64, 2>();
     hipLaunchKernelGGL((gemm_dma<128, 128, 2, 2, 64, 2, occ>), dim3((unsigned) (nt_m * nt_n), (unsigned) splits),
                        dim3(256), 0, s, q, nt_m, nt_n);
-}
-static hipError_t run_dma_splitk(const GemmParams & p, int splits, void * ws, hipStream_t s) {
-    launch_dma_splitk_parts(p, splits, ws, s);
-    launch_reduce(p, (const float *) ws, splits, s);
-    return hipGetLastError();
 }
 
 // Tile shape of the bf16 x bf16 DMA path, chosen so the grid fills the 256 CUs
@@ -2270,6 +2266,14 @@ static DmaPlan dma_plan(const GemmParams & p, size_t ws_bytes) {
     return best;
 }
 
+// The slices of a plan with more than one; a reduce in slice order follows
+// (launch_reduce, or launch_gemm_rowpost's with the row ops).
+static void launch_dma_parts(const GemmParams & p, const DmaPlan & d, void * ws, hipStream_t s) {
+    if (d.tile == 256) launch_pipe_parts<256, 256, 4, 2, 4, kSchedPingPong, 32>(p, d.splits, ws, s);
+    else if (d.tile == 192) launch_pipe_parts<192, 192, 2, 2, 3, kSchedProducer, 64>(p, d.splits, ws, s);
+    else launch_dma_splitk_parts(p, d.splits, ws, s);
+}
+
 static bool dispatch_dma(const GemmParams & p, void * ws, size_t ws_bytes, hipStream_t s, hipError_t & err) {
     if (p.K % 32 != 0) return false;
     if (tiles_of(p, 256, 256) >= 256) {
@@ -2284,17 +2288,20 @@ static bool dispatch_dma(const GemmParams & p, void * ws, size_t ws_bytes, hipSt
     if (p.K % 64 != 0) return false;
     if (!ws || ((uintptr_t) ws & 15)) ws_bytes = 0;
     const DmaPlan d = dma_plan(p, ws_bytes);
-    if (d.tile == 256)
-        err = d.splits > 1 ? launch_pipe_splitk<256, 256, 4, 2, 4, kSchedPingPong, 32>(p, d.splits, ws, s)
-                           : run_dma_pipe<256, 256, 4, 2, 4, 32, 3, kSchedPingPong>(p, s);
-    else if (d.tile == 192)
+    if (d.splits > 1) {
+        launch_dma_parts(p, d, ws, s);
+        launch_reduce(p, (const float *) ws, d.splits, s);
+        err = hipGetLastError();
+    } else if (d.tile == 256) {
+        err = run_dma_pipe<256, 256, 4, 2, 4, 32, 3, kSchedPingPong>(p, s);
+    } else if (d.tile == 192) {
         // K steps of 64 in a 3-stage ring (144 KB): half the barriers and
         // waits per K of the 4-stage BK 32 ring, same bits.  3072^2 55.6
         // against 64.0 us, FFN-down (K 14336) 234 against 280.
-        err = d.splits > 1 ? launch_pipe_splitk<192, 192, 2, 2, 3, kSchedProducer, 64>(p, d.splits, ws, s)
-                           : run_dma_pipe<192, 192, 2, 2, 3, 64, 3, kSchedProducer, 64>(p, s);
-    else
-        err = d.splits > 1 ? run_dma_splitk(p, d.splits, ws, s) : run_dma<128, 128, 2, 2, 64, 2>(p, s);
+        err = run_dma_pipe<192, 192, 2, 2, 3, 64, 3, kSchedProducer, 64>(p, s);
+    } else {
+        err = run_dma<128, 128, 2, 2, 64, 2>(p, s);
+    }
     return true;
 }
 
@@ -2491,22 +2498,38 @@ hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStre
         !p.vec_out || E == kEpiF32 || !a.ws || !aligned16(a.ws))
         return hipErrorNotSupported;
     if (a.w_tiled && (p.M % 16 != 0 || p.K % 32 != 0)) return hipErrorNotSupported;
-    // More than 64 tokens: only the products that dispatch_dma runs as the
-    // K-sliced 128 x 128 GEMM (its partial planes are the reduce's layout).
-    const bool dma = a.N > 64;
+    // The kernel and K slices that launch_gemm takes for the product, so that
+    // its sums are the same with the row ops and without.  More than 64 tokens:
+    // the products that dispatch_dma cuts along K (their planes are the
+    // reduce's layout; an unsplit one would only write its output wider).
+    //
+    // Two few-token products sum in another f32 order here than alone:
+    // gemm_row16's at 2 to 48 tokens, and those of gemm_skinny_wk (tiled weights
+    // of 12288 features or more).  Their gain is the reduce launch that they do
+    // without, and here a reduce follows anyway.  LINEAR + LayerNorm, weights
+    // from HBM, in us, gemm_row16 into one plane against the K slices: tiled
+    // 3072 x 48 x 3072 18.8 / 15.2, 2048 x 48 x 2048 14.2 / 12.6; row-major
+    // 3072 x 8 x 3072 13.9 / 12.9, 1024 x 48 x 1024 10.2 / 8.7.  At one token
+    // it is the better one or close (tiled 3072 x 1 x 3072 11.4 / 15.4, 3072 x
+    // 1 x 14336 26.4 / 24.9; row-major 3072 x 1 x 3072 12.4 / 12.2).
+    const bool xf32 = a.x_type == WAMX_TYPE_F32, dma = a.N > 64;
+    const bool row16 = p.N == 1 && row16_ok(p, xf32, a.w_tiled);
     int splits = 1, ks = 0, waves = 0;
     GenPlan gp{};
+    DmaPlan dp{};
     if (dma) {
-        if (a.w_tiled || a.x_type != WAMX_TYPE_BF16 || p.K % 64 != 0 || tiles_of(p, 256, 256) >= 256 ||
-            tiles_of(p, 192, 192) >= 192)
-            return hipErrorNotSupported;
-        splits = dma_splitk_plan(p, a.ws_bytes);
+        if (a.w_tiled || xf32 || p.K % 64 != 0 || tiles_of(p, 256, 256) >= 256) return hipErrorNotSupported;
+        dp = dma_plan(p, a.ws_bytes);
+        splits = dp.splits;
         if (splits <= 1) return hipErrorNotSupported;
+    } else if (!a.w_tiled && skinny_workspace_bytes(p.M, p.N, p.K) > a.ws_bytes) {
+        return hipErrorNotSupported;
+    } else if (row16) {
+        // One plane.
     } else if (a.w_tiled) {
         skinny_tiled_plan(p.M, p.N, p.K, splits, ks, waves);
     } else {
-        if (skinny_workspace_bytes(p.M, p.N, p.K) > a.ws_bytes) return hipErrorNotSupported;
-        gp = gen_plan(p, true, a.x_type == WAMX_TYPE_BF16, 1, a.ws_bytes);
+        gp = gen_plan(p, true, !xf32, 1, a.ws_bytes);
         splits = gp.splits;
     }
     if ((size_t) splits * p.N * p.M * sizeof(float) > a.ws_bytes) return hipErrorNotSupported;
@@ -2585,12 +2608,15 @@ hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStre
 
     const float * part = (const float *) a.ws;
     if (dma) {
-        launch_dma_splitk_parts(p, splits, a.ws, s);
+        launch_dma_parts(p, dp, a.ws, s);
+    } else if (row16) {
+        const hipError_t e = run_row16(plane_params(p, a.ws), xf32, a.w_tiled, Chain{}, s);
+        if (e != hipSuccess) return e;
     } else if (a.w_tiled) {
         allow_skinny_lds();
-        launch_skinny_part(p, a.x_type == WAMX_TYPE_F32, (float *) a.ws, splits, ks, waves, s);
+        launch_skinny_part(p, xf32, (float *) a.ws, splits, ks, waves, s);
     } else {
-        launch_gen_part(p, true, a.x_type == WAMX_TYPE_BF16, (float *) a.ws, gp, 1, s);
+        launch_gen_part(p, true, !xf32, (float *) a.ws, gp, 1, s);
     }
     const dim3 grid((unsigned) p.N, (unsigned) nseg), block((unsigned) nchunk);
 #define WAMX_ROW(EK, PK) hipLaunchKernelGGL((skinny_reduce_row<EK, PK>), grid, block, 0, s, p, part, splits, d)
