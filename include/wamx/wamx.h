@@ -461,6 +461,10 @@ WAMX_API void           wamx_gallocr_free(wamx_gallocr_t galloc);
  * (uid, node count and tensor addresses) was computed before; set
  * WAMX_DISABLE_HIP_GRAPHS=1 to launch eagerly every time. */
 WAMX_API wamx_status wamx_backend_graph_compute(wamx_backend_t backend, wamx_cgraph * g);
+/* Nodes that the launch of an earlier node computed too (a product's row ops
+ * or element-wise nodes), since the backend was made; a replayed graph counts
+ * once, when it is captured. */
+WAMX_API int64_t     wamx_backend_fused_nodes(wamx_backend_t backend);
 WAMX_API bool        wamx_backend_supports_op(wamx_backend_t backend, const wamx_tensor * op);
 
 /* ---------------------------------------------------------------------------

@@ -195,7 +195,9 @@ def _linear_norm(wx, be, rng, M, K, T, tiled, epi):
                      (sc, bf(1 + 0.1 * rng.standard_normal(M))), (sh, bf(0.1 * rng.standard_normal(M))),
                      (gate, (0.5 * rng.standard_normal(M)).astype(np.float32))):
             g.set(t, a)
+        before = lib.wamx_backend_fused_nodes(be.ptr)
         g.compute(n)
+        assert lib.wamx_backend_fused_nodes(be.ptr) - before == 1  # the norm went along
         got = [g.get(t, np.uint16, (T, M)) for t in (y, n)]
         alone, norm = be.empty(T * M * 2), be.empty(T * M * 2)
         op = lib.wamx_op_linear_tiled if tiled else lib.wamx_op_linear

@@ -66,6 +66,7 @@ struct wamx_backend {
     bool fuse_rows = true;       // split-K reduce + consuming row op in one launch
     bool fuse_norm_mod_f32 = true;       // F32 NORM -> MUL -> ADD -> ADD as one launch
     bool fuse_gated_residual_f32 = true; // F32 MUL -> ADD as one launch
+    int64_t fused_nodes = 0;     // nodes that an earlier node's launch computed too
     std::unordered_map<uint64_t, GraphCacheEntry> graphs;
 };
 
@@ -1232,6 +1233,7 @@ static wamx_status run_nodes(wamx_backend * be, wamx_cgraph * g) {
             }
             done[i] = 1;
         }
+        be->fused_nodes += nm - 1;
         if (two)
             for (int m = 0; m < nm; ++m)
                 if (signal[members[m]]) hipEventRecord(be->events[slot[members[m]]], be->cs);
@@ -1714,6 +1716,7 @@ wamx_status wamx_backend_graph_compute(wamx_backend_t be, wamx_cgraph * g) {
     return graph_compute_impl(be, g);
 }
 bool wamx_backend_supports_op(wamx_backend_t, const wamx_tensor * op) { return op && supports(op); }
+int64_t wamx_backend_fused_nodes(wamx_backend_t be) { return be ? be->fused_nodes : 0; }
 
 // --- single-op entry points ---------------------------------------------
 #define WAMX_LAUNCH(expr)                                                                  \

@@ -203,6 +203,7 @@ def load(path: str | os.PathLike | None = None) -> C.CDLL:
         "wamx_graph_assign_uid": (None, [vp]),
         "wamx_graph_uid": (C.c_uint64, [vp]),
         "wamx_backend_supports_op": (C.c_bool, [vp, TensorP]),
+        "wamx_backend_fused_nodes": (i64, [vp]),
         "wamx_backend_graph_compute": (C.c_int, [vp, vp]),
         "wamx_backend_alloc_ctx_tensors": (vp, [vp, vp]),
         "wamx_backend_alloc_ctx_tensors_from_buft": (vp, [vp, vp]),
