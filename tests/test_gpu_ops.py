@@ -534,8 +534,10 @@ def test_empty_and_refused_sizes(wx, be):
     assert np.array_equal(y.download(np.uint16, (4096,)), sentinel)
 
 
-# The K-sliced 256 x 256 and 192 x 192 tiles (dma_plan), whole and with ragged
-# edges, and their f32 outputs.
+# Large tiles (dma_plan), whole and with ragged edges, and their f32 outputs:
+# 256 x 256 in 2, 4 and 8 slices (with f32 activations, whose bf16 copy takes
+# part of the workspace, 192 x 192 in 1, 2 and 256 x 256 in 8) and unsplit,
+# 128 x 128 and 192 x 192 unsplit.
 @pytest.mark.parametrize("M,N,K", [(3072, 2048, 14336), (3072, 1000, 14336), (3000, 500, 14336), (14336, 1000, 512),
                                    (9216, 1030, 256), (4096, 1500, 4096)])
 @pytest.mark.parametrize("xt", ["f32", "bf16"])
@@ -550,9 +552,11 @@ def test_mul_mat_sliced_large_tiles_integers_exact(wx, be, M, N, K, xt):
     assert np.array_equal(gpu_mul_mat(wx, be, bf16(w), xin, wx.TYPE_BF16), bf16(ref))
 
 
-# One launch for few tokens (gemm_row16): K below, at and past a round of the
-# waves' 32-column tiles and not a multiple of 32 (row-major), features below
-# and past 16, 1 to 48 tokens, both weight layouts and activation types.
+# One launch for few tokens on row-major weights (gemm_row16): K below, at and
+# past a round of the waves' 32-column tiles and not a multiple of 32, features
+# below and past 16, 1 to 48 tokens, both activation types.  (8, 48, 2056) and,
+# with f32 activations, (1024, 48, 1024) and (4096, 32, 2048) are past its bound
+# and run gemm_gen.
 @pytest.mark.parametrize("M,N,K", [(3072, 1, 3072), (1024, 48, 1024), (16, 17, 32), (40, 5, 72), (1000, 33, 264),
                                    (2000, 16, 1048), (4096, 32, 2048), (8, 48, 2056)])
 @pytest.mark.parametrize("xt", ["f32", "bf16"])
@@ -565,3 +569,27 @@ def test_few_tokens_one_launch_integers_exact(wx, be, M, N, K, xt):
     xin = x if xt == "f32" else bf16(x)
     assert np.array_equal(gpu_mul_mat(wx, be, bf16(w), xin, wx.TYPE_F32), ref)
     assert np.array_equal(gpu_mul_mat(wx, be, bf16(w), xin, wx.TYPE_BF16), bf16(ref))
+
+
+# The tiles and slices that the shapes above leave out: 192 x 192 in 4 and 16
+# slices, 128 x 128 in 6 and 16, and one 256 x 256 tile or more per CU; feature
+# counts that bf16 outputs cannot store in 16-byte chunks (f32 ones do not need
+# to) at each tile.
+@pytest.mark.parametrize("M,N,K", [(9216, 192, 3072), (3072, 192, 14336), (3072, 384, 3072), (3072, 65, 14336),
+                                   (14336, 3072, 256), (9212, 190, 3072), (3004, 3000, 256), (14332, 3001, 256)])
+def test_mul_mat_every_tile_integers_exact(wx, be, M, N, K):
+    print(f"mul_mat every tile M={M} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    w = rng.integers(-4, 5, (M, K)).astype(np.float32)
+    x = rng.integers(-4, 5, (N, K)).astype(np.float32)
+    ref = x @ w.T  # exact in f32: sums below 2^24
+    assert np.array_equal(gpu_mul_mat(wx, be, bf16(w), bf16(x), wx.TYPE_F32), ref)
+    assert np.array_equal(gpu_mul_mat(wx, be, bf16(w), bf16(x), wx.TYPE_BF16), bf16(ref))
+
+
+# f32 activations on row-major weights within gemm_row16's bound (200 KB copied
+# per CU) for two and three token tiles.
+@pytest.mark.parametrize("M,N,K", [(512, 32, 512), (512, 48, 512), (520, 20, 520), (264, 33, 744)])
+def test_few_tokens_one_launch_f32_activations_exact(wx, be, M, N, K):
+    assert -(-M // 4096) * K * 32 / 1024 * (1 + 2.5 * -(-N // 16)) <= 200
+    test_few_tokens_one_launch_integers_exact(wx, be, M, N, K, "f32")

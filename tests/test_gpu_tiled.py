@@ -109,8 +109,9 @@ def test_layout_and_conversions(wx, be, rng):
         B.close()
 
 
-# One-token shapes (the state token's projections) run the K-split plans of
-# grids in rounds of 64 workgroups; the rest in rounds of 256.
+# 3072 x 48 x 14336 and 9216 x 48 x 3072 run the K-split plans
+# (gemm_skinny_tiled and a reduce), the rest one launch (gemm_row16); the
+# tests below hold each kernel at every token tile and activation type.
 @pytest.mark.parametrize("M,K,N", [(3072, 3072, 48), (9216, 3072, 48), (3072, 14336, 48), (14336, 3072, 1),
                                    (3072, 3072, 1), (9216, 3072, 1), (3072, 14336, 1),
                                    (3072, 3072, 17), (128, 96, 5)])
@@ -139,8 +140,9 @@ def test_integer_products_exact(wx, be, M, K, N):
 @pytest.mark.parametrize("M,K,N", [(3072, 3072, 48), (3072, 3072, 1), (9216, 3072, 1), (3072, 14336, 1),
                                    (3072, 3072, 17), (128, 96, 5)])
 def test_integer_products_f32_activations_exact(wx, be, M, K, N):
-    """Tiled weights times f32 activations (gemm_skinny_tiled's f32 form, which
-    rounds each activation to bf16 as it stages it). Small integers survive
+    """Tiled weights times f32 activations, each rounded to bf16 on its way
+    (in gemm_skinny_tiled's staging at 3072 x 48 x 3072 and 3072 x 1 x 14336,
+    in gemm_row16's registers at the others). Small integers survive
     that rounding, and their fp32 sums are exact, so the output must equal
     x @ w.T exactly."""
     print(f"tiled integer product, f32 activations, M={M} K={K} N={N}", flush=True)
@@ -160,6 +162,42 @@ def test_integer_products_f32_activations_exact(wx, be, M, K, N):
             B.compute(y)
             got = B.get(y, np.float32, (N, M))
             assert np.array_equal(got.astype(np.int64), x @ w.T), f"launch {rep}"
+    finally:
+        B.close()
+
+
+# M, K, N past and within gemm_row16's bound (600 KB copied per CU), for one to
+# four token tiles of 16; a product that gemm_skinny_wk takes has bf16 output.
+SPLIT = [("bf16", 14336, 4096, 1), ("bf16", 3072, 14336, 8), ("bf16", 9216, 3072, 17), ("bf16", 9216, 3072, 33),
+         ("bf16", 1024, 1024, 64), ("f32", 9216, 4096, 1), ("f32", 9216, 3072, 8), ("f32", 9216, 3072, 17),
+         ("f32", 3072, 3072, 40), ("f32", 1024, 1024, 64)]
+ONE = [("bf16", 3072, 3072, 1), ("bf16", 9216, 3072, 8), ("bf16", 2048, 2048, 20), ("bf16", 1040, 1056, 48),
+       ("bf16", 16, 32, 33), ("f32", 3072, 3072, 1), ("f32", 1024, 1024, 16), ("f32", 2048, 2048, 20),
+       ("f32", 528, 544, 48), ("f32", 16, 32, 33)]
+
+
+@pytest.mark.parametrize("xt,M,K,N", SPLIT + ONE)
+def test_integer_products_each_kernel_exact(wx, be, xt, M, K, N):
+    one = (xt, M, K, N) in ONE
+    nt, f = -(-N // 16), 2.5 if xt == "f32" else 1
+    kb = -(-M // 4096) * K * 32 / 1024 * (1 + f * (0.25 if N == 1 else nt))
+    assert one == (N <= 48 and kb <= 600)
+    print(f"tiled integer product M={M} K={K} N={N} x={xt} {'one launch' if one else 'K slices'}", flush=True)
+    lib = be.lib
+    rng = np.random.default_rng(M + 3 * K + 7 * N)
+    w = rng.integers(-4, 5, (M, K)).astype(np.float32)
+    x = rng.integers(-4, 5, (N, K)).astype(np.float32)
+    B = Bufs(wx, be)
+    try:
+        wt = B.tiled(K, M)
+        xin = B.plain(wx.TYPE_F32 if xt == "f32" else wx.TYPE_BF16, K, N)
+        y = lib.wamx_mul_mat(B.pctx, wt, xin)
+        B.alloc()
+        assert wt.contents.extra
+        B.set(wt, wx.f32_to_bf16(w))
+        B.set(xin, x if xt == "f32" else wx.f32_to_bf16(x))
+        B.compute(y)
+        assert np.array_equal(B.get(y, np.float32, (N, M)), x @ w.T)  # exact in f32: sums below 2^24
     finally:
         B.close()
 
