@@ -7,9 +7,10 @@ plus the same reduce, with chunk-major Q/K and V^T destinations.  The fused grap
 must produce the same bits as the standalone ops launched one at a time
 (wamx_op_linear, wamx_op_norm_modulation_bf16 / wamx_op_layer_norm_bf16,
 wamx_op_qk_norm_rope and a host transpose for V^T), which the per-op tests
-hold to the oracle.  Products of 2 to 48 tokens that run in one launch when
-alone sum in another f32 order there: the row op is the same bits on the fused
-product, and the two products differ by no more than the order of the sum.
+hold to the oracle.  Products of few tokens that run in one launch when alone
+(on tiled weights, or 2 to 48 tokens) sum in another f32 order there: the row
+op is the same bits on the fused product, and the two products differ by no
+more than the order of the sum.
 """
 from __future__ import annotations
 
@@ -217,10 +218,10 @@ def _linear_norm(wx, be, rng, M, K, T, tiled, epi):
         lib.wamx_free(tctx)
 
 
-# One token in one launch per product (tiled and row-major), and the tiles and
-# K slices of each kind above 64 tokens (3072 x 14336: 16 slices of 192 x 192
+# One token in one launch (row-major), K slices of tiled weights, and the tiles
+# and K slices of each kind above 64 tokens (3072 x 14336: 16 slices of 192 x 192
 # at 192 tokens, 8 of them at 384, 8 of 256 x 256 at 512; 16 of 128 x 128 at 65).
-@pytest.mark.parametrize("M,K,T,tiled", [(3072, 3072, 1, True), (3072, 14336, 1, True), (1024, 1024, 1, False),
+@pytest.mark.parametrize("M,K,T,tiled", [(1024, 1024, 1, False), (3072, 14336, 48, True), (3072, 4096, 64, True),
                                          (3072, 14336, 65, False), (3072, 14336, 192, False),
                                          (3072, 14336, 384, False), (3072, 14336, 512, False)])
 def test_linear_then_norm_sums_as_the_product_alone(wx, be, rng, M, K, T, tiled):
@@ -236,10 +237,10 @@ def test_qkv_split_many_tokens_is_bit_exact(wx, be, rng, T):
     test_qkv_split_is_bit_exact(wx, be, rng, T)
 
 
-@pytest.mark.parametrize("M,K,T,tiled", [(3072, 3072, 48, True), (2048, 2048, 20, True), (3072, 3072, 8, False),
-                                         (1024, 1024, 48, False)])
+@pytest.mark.parametrize("M,K,T,tiled", [(3072, 3072, 1, True), (3072, 14336, 1, True), (3072, 3072, 48, True),
+                                         (2048, 2048, 20, True), (3072, 3072, 8, False), (1024, 1024, 48, False)])
 def test_few_token_products_sum_in_another_order_alone(wx, be, rng, M, K, T, tiled):
-    """Products of 2 to 48 tokens that take one launch when alone: both sums
+    """Products that take one launch when alone and K slices before a row op: both sums
     are within K f32 roundings (2^-23, a truncating adder's) of the exact one
     and rounded to bf16 once (2^-8); the norm is that of the fused product."""
     print(f"fusion few tokens {M}x{T}x{K} tiled={tiled}", flush=True)

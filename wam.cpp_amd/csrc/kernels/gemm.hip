@@ -2504,16 +2504,18 @@ hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStre
     // reduce's layout; an unsplit one would only write its output wider).
     //
     // Two few-token products sum in another f32 order here than alone:
-    // gemm_row16's at 2 to 48 tokens, and those of gemm_skinny_wk (tiled weights
-    // of 12288 features or more).  Their gain is the reduce launch that they do
-    // without, and here a reduce follows anyway.  LINEAR + LayerNorm, weights
-    // from HBM, in us, gemm_row16 into one plane against the K slices: tiled
-    // 3072 x 48 x 3072 18.8 / 15.2, 2048 x 48 x 2048 14.2 / 12.6; row-major
-    // 3072 x 8 x 3072 13.9 / 12.9, 1024 x 48 x 1024 10.2 / 8.7.  At one token
-    // it is the better one or close (tiled 3072 x 1 x 3072 11.4 / 15.4, 3072 x
-    // 1 x 14336 26.4 / 24.9; row-major 3072 x 1 x 3072 12.4 / 12.2).
+    // gemm_row16's on tiled weights or at 2 to 48 tokens, and those of
+    // gemm_skinny_wk (tiled weights of 12288 features or more).  Their gain is
+    // the reduce launch that they do without, and here a reduce follows anyway.
+    // LINEAR + LayerNorm, weights from HBM, in us, gemm_row16 into one plane
+    // against the K slices: tiled 3072 x 48 x 3072 18.8 / 15.2, 2048 x 48 x 2048
+    // 14.2 / 12.6, 3072 x 1 x 14336 26.4 / 24.9; row-major 3072 x 8 x 3072 13.9 /
+    // 12.9, 1024 x 48 x 1024 10.2 / 8.7.  Tiled 3072 x 1 x 3072 is 11.4 / 15.4,
+    // but beside the visual tokens' kernels the whole action chunk was slower
+    // with it (83.68 against 83.53 ms, six runs each): the slices of the state
+    // token's products take a quarter of the CUs (skinny_tiled_plan).
     const bool xf32 = a.x_type == WAMX_TYPE_F32, dma = a.N > 64;
-    const bool row16 = p.N == 1 && row16_ok(p, xf32, a.w_tiled);
+    const bool row16 = p.N == 1 && !a.w_tiled && row16_ok(p, xf32, false);
     int splits = 1, ks = 0, waves = 0;
     GenPlan gp{};
     DmaPlan dp{};
@@ -2524,11 +2526,9 @@ hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStre
         if (splits <= 1) return hipErrorNotSupported;
     } else if (!a.w_tiled && skinny_workspace_bytes(p.M, p.N, p.K) > a.ws_bytes) {
         return hipErrorNotSupported;
-    } else if (row16) {
-        // One plane.
     } else if (a.w_tiled) {
         skinny_tiled_plan(p.M, p.N, p.K, splits, ks, waves);
-    } else {
+    } else if (!row16) {  // which writes one plane
         gp = gen_plan(p, true, !xf32, 1, a.ws_bytes);
         splits = gp.splits;
     }
@@ -2610,7 +2610,7 @@ hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStre
     if (dma) {
         launch_dma_parts(p, dp, a.ws, s);
     } else if (row16) {
-        const hipError_t e = run_row16(plane_params(p, a.ws), xf32, a.w_tiled, Chain{}, s);
+        const hipError_t e = run_row16(plane_params(p, a.ws), xf32, false, Chain{}, s);
         if (e != hipSuccess) return e;
     } else if (a.w_tiled) {
         allow_skinny_lds();
