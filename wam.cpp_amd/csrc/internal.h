@@ -23,8 +23,8 @@ const char * check_conv_2d(const wamx_tensor * t);
 
 // ---------------------------------------------------------------------------
 // GEMM: y[b][n][m] = sum_k w[b/r][m][k] * x[b][n][k]  (the ggml MUL_MAT layout:
-// both operands K-contiguous, "NT").  w is bf16 (or f32 for the SIMT path),
-// x is bf16 or f32 (rounded to bf16 on load when w is bf16).
+// both operands K-contiguous, "NT").  w is bf16 or f32, x is bf16 or f32
+// (rounded to bf16 on load when w is bf16; products in f32 when w is f32).
 // ---------------------------------------------------------------------------
 struct GemmArgs {
     const void * w = nullptr;
@@ -44,7 +44,7 @@ struct GemmArgs {
     const void * res = nullptr;              // bf16 [N][ldres]
     int64_t ldres = 0;
     const float * gate = nullptr;            // f32 [M]
-    void * ws = nullptr;                     // K-split partials of the skinny path
+    void * ws = nullptr;                     // K-split partials, rounded activations
     size_t ws_bytes = 0;
     bool w_tiled = false;                    // w in the MFMA-tiled layout (launch_tile_weights)
 };
@@ -57,7 +57,8 @@ hipError_t launch_tile_weights(const void * src, void * dst, int64_t M, int64_t 
 bool tensor_is_tiled(const wamx_tensor * t);
 // Writes the row-major device array src into t, tiling it when t is tiled.
 hipError_t tensor_set_from_device(wamx_tensor * t, const void * src, hipStream_t s);
-// Workspace the skinny path needs for an M x N x K product (0 when unsplit).
+// Workspace below which a few-token product on row-major bf16 weights is
+// refused (0: none), whatever its kernel writes.
 size_t skinny_workspace_bytes(int64_t M, int64_t N, int64_t K);
 // Workspace of a backend: K-split GEMM and key-split attention partials.
 constexpr size_t kBackendWorkspaceBytes = 64ull << 20;
@@ -121,9 +122,10 @@ struct RowPost {
 // when the product or the row op does not fit that path.
 hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStream_t s);
 
-// Element-wise nodes that follow a product, applied by its last launch: v is the product's value as its node stores it, each stage's result
-// is rounded to the output type, and every node's output is written (but one
-// whose tensor the next stage overwrites in place).
+// Element-wise nodes that follow a product, applied by its last launch: v is
+// the product's value as its node stores it, each stage's result is rounded to
+// the output type, and every node's output is written (but one whose tensor the
+// next stage overwrites in place).
 enum { kStageAddRow = 1, kStageAdd, kStageMulRow, kStageMul, kStageGelu, kStageBiasGelu, kStageGated };
 struct ChainStage {
     int32_t kind = 0;

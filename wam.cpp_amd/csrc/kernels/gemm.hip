@@ -6,9 +6,13 @@
 // src/models/gwp05/artifact.cpp:115-116), x the activation (bf16, or f32
 // rounded to bf16 on load: ggml converts src1 to the weight's vec-dot type).
 //
-// Three kernels:
-//  * gemm_tile   — MFMA 32x32x16 bf16, LDS double-buffered 128x128x64 tiles,
-//                  128-bit global loads, for token counts above 64.
+// Products:
+//  * gemm_dma_pipe, gemm_dma — bf16 operands, more than 64 tokens: operands copied
+//                  straight into an LDS ring, tiles of 128 x 128 to 256 x 256
+//                  (dma_plan), in K slices where the tiles leave CUs idle.
+//  * gemm_tile   — f32, unaligned or batched activations above 64 tokens:
+//                  MFMA 32x32x16 bf16, LDS double-buffered 128x128x64 tiles
+//                  staged through registers.
 //  * gemm_skinny_tiled, gemm_skinny_wk — N <= 64 tokens (the 48-token action
 //                  expert) on tiled weights: HBM-bound weight streaming with
 //                  MFMA 16x16x32.
@@ -16,6 +20,9 @@
 //  * gemm_gen    — N <= 64 tokens on row-major weights, batches and any
 //                  alignment included, and f32 weights (the f32 reference
 //                  profile, generic MUL_MAT) on f32 MFMA 16x16x4.
+// Reduces of the K slices' f32 planes: gemm_skinny_reduce (with the product's
+// epilogue), skinny_reduce_row (and the row ops after it), gemm_reduce_chain
+// (and the element-wise nodes after it).
 #include "../internal.h"
 #include "device.h"
 #include "rowops.h"
