@@ -2521,6 +2521,8 @@ hipError_t launch_gemm_rowpost(const GemmArgs & a, const RowPost & post, hipStre
     // but beside the visual tokens' kernels the whole action chunk was slower
     // with it (83.68 against 83.53 ms, six runs each): the slices of the state
     // token's products take a quarter of the CUs (skinny_tiled_plan).
+    // One token on row-major weights measures alike (3072 x 1 x 3072 12.4 / 12.2)
+    // and takes it here too.
     const bool xf32 = a.x_type == WAMX_TYPE_F32, dma = a.N > 64;
     const bool row16 = p.N == 1 && !a.w_tiled && row16_ok(p, xf32, false);
     int splits = 1, ks = 0, waves = 0;
